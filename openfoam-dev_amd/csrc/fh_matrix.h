@@ -5,6 +5,7 @@
 
 #include "fh_kernels.h"
 #include "fh_solver_kernels.h"
+#include "fh_tile_march.h"
 #include "fh_tile_sweep.h"
 
 #include <algorithm>
@@ -102,6 +103,11 @@ struct fh_matrix
     fh::DBuf<unsigned int> d_tileFlags;
     fh::DBuf<unsigned long long> d_tileTicket;
     unsigned long long tileTicketBase = 0, tileEpoch = 0;
+    // marching sweeps of the global DIC / DILU (hex boxes): packed pass
+    // coefficients and halos; err: set when a wait expired
+    fh::MarchBufs<double> march64;
+    fh::MarchBufs<float> march32;
+    fh::DBuf<unsigned int> d_marchErr;
 
     // live timing of chosen kernels inside the solver loops: a pair of HIP
     // events around every launch of a kernel whose FH_KERNEL_* bit is set in

@@ -92,6 +92,8 @@ void matrix_init(fh_matrix* M, fh_mesh* mesh, hipStream_t shared)
         M->d_tileTicket.alloc(1);
         FH_HIP(hipMemsetAsync(M->d_tileFlags.p, 0, M->d_tileFlags.bytes(), M->stream));
         FH_HIP(hipMemsetAsync(M->d_tileTicket.p, 0, M->d_tileTicket.bytes(), M->stream));
+        M->d_marchErr.alloc(1);
+        FH_HIP(hipMemsetAsync(M->d_marchErr.p, 0, M->d_marchErr.bytes(), M->stream));
     }
     FH_HIP(hipStreamSynchronize(M->stream));
     M->epoch = 0;
@@ -181,6 +183,7 @@ void matrix_coeffs_updated(fh_matrix* M)
     M->padValid = false;
     M->halfState = 0;
     M->coarseState = 0;
+    M->march64.kind = M->march32.kind = -1;
     for (int i = 0; i < 5; i++) M->rDValid[i] = M->rD32Valid[i] = false;
     gamg_invalidate(M);
 }
@@ -549,37 +552,75 @@ template<> void sweep_t<float>(fh_matrix* M, int kind, const SweepData<float>& d
     sweep_f(M, kind, d, st, local);
 }
 
-// One global DIC / DILU pass on a box from packed coefficients (partials:
-// the backward pass also sums w*x into one partial per tile); returns the
-// partial count.  One-wavefront 8 x 8 x 16 tiles unless the workgroup
-// kernel over 16 x 16 x bz tiles is asked for (FOAMHIP_BOX_SWEEP=wide).
+template<class T> static MarchBufs<T>& march_bufs(fh_matrix* M);
+template<> MarchBufs<double>& march_bufs<double>(fh_matrix* M) { return M->march64; }
+template<> MarchBufs<float>& march_bufs<float>(fh_matrix* M) { return M->march32; }
+
+// the marching sweeps' coefficients of factor `which` (both passes) and
+// their halos
 template<class T>
-static int32_t box_precond_pass(fh_matrix* M, bool backward, const SweepData<T>& d0,
+static MarchBufs<T>& ensure_march(fh_matrix* M, int which, const T* rD)
+{
+    MarchBufs<T>& b = march_bufs<T>(M);
+    const TileView G = M->tile_view(16, 8);
+    if (b.kind != which)
+    {
+        for (int bwd = 0; bwd < 2; bwd++)
+        {
+            SweepData<T> d{};
+            set_sweep_dirs<T>(M, d, bwd != 0);
+            launch_march_pack<T>(bwd != 0, G, rD, d.dir, d.dirShift != 0, b, M->stream);
+        }
+        b.kind = which;
+    }
+    march_prepare_halo<T>(G, b, M->stream);
+    return b;
+}
+
+// One global DIC / DILU pass (factor `which`) on a box from packed
+// coefficients (partials: the backward pass also sums w*x into one partial
+// per pencil or tile); returns the partial count.  The marching pencils
+// where the box has planes enough for them, the one-wavefront 8 x 8 x 16
+// tiles otherwise; FOAMHIP_BOX_SWEEP=wave or wide asks for those tiles or
+// for the workgroup kernel over 16 x 16 x bz tiles.
+template<class T>
+static int32_t box_precond_pass(fh_matrix* M, int which, bool backward, const SweepData<T>& d0,
                                 double* partials, DevState* st,
                                 const FusedFinalize& F = FusedFinalize(), bool* fused = nullptr)
 {
     SweepData<T> d = d0;
-    set_sweep_dirs<T>(M, d, backward);
     if (backward && partials)
     {
         d.dotR = d.x;
         d.partials = partials;
     }
-    static const bool wide = [] {
+    static const int forced = [] {
         const char* e = std::getenv("FOAMHIP_BOX_SWEEP");
-        return e && std::strcmp(e, "wide") == 0;
+        return !e ? 0 : std::strcmp(e, "wide") == 0 ? 1 : std::strcmp(e, "wave") == 0 ? 2 : 0;
     }();
-    if (!wide)
+    if (forced != 1)
     {
         TileSync ts = M->tile_sync();
         const bool fuse = backward && partials && F.counter;
-        const int32_t n = launch_sweep_wave<T>(backward, M->tile_view(16, 8), d, ts, st,
-                                               M->stream, fuse ? F : FusedFinalize());
+        const FusedFinalize& Ff = fuse ? F : FusedFinalize();
+        int32_t n;
+        if (forced == 0 && march_fits(M->mesh->boxNx, M->mesh->boxNy, M->mesh->boxNz, sizeof(T)))
+        {
+            const MarchBufs<T>& b = ensure_march<T>(M, which, d.rD);
+            n = launch_sweep_march<T>(backward, M->tile_view(16, 8), d, b, ts, M->d_marchErr.p,
+                                      st, M->stream, Ff);
+        }
+        else
+        {
+            set_sweep_dirs<T>(M, d, backward);
+            n = launch_sweep_wave<T>(backward, M->tile_view(16, 8), d, ts, st, M->stream, Ff);
+        }
         if (fused) *fused = fuse;
         M->tileTicketBase = ts.ticketBase;
         M->tileEpoch = ts.epoch;
         return n;
     }
+    set_sweep_dirs<T>(M, d, backward);
     sweep_t<T>(M, backward ? SWEEP_PRECOND_BWD : SWEEP_PRECOND_FWD, d, st, false);
     const TileView G = M->tile_view(pre_bz<T>(M));
     return G.nTI*G.nTJ*G.nTK;
@@ -719,8 +760,8 @@ int32_t apply_precond(fh_matrix* M, int precon, const T* r, T* w, double* partia
     {
         // global sweeps on a box: packed coefficients, and the backward pass
         // sums w*r per tile
-        box_precond_pass<T>(M, false, d, nullptr, st);
-        return box_precond_pass<T>(M, true, d, partials, st, F, fused);
+        box_precond_pass<T>(M, which, false, d, nullptr, st);
+        return box_precond_pass<T>(M, which, true, d, partials, st, F, fused);
     }
     sweep_t<T>(M, SWEEP_PRECOND_FWD, d, st, local);
     sweep_t<T>(M, transpose && dilu ? SWEEP_PRECOND_BWD_T : SWEEP_PRECOND_BWD, d, st, local);
@@ -912,6 +953,20 @@ void fill_perf(fh_matrix* M, fh_perf* perf, const char* name)
 
 void check_sweep_errors(fh_matrix* M)
 {
+    if (M->march64.haloReady || M->march32.haloReady)
+    {
+        unsigned int e = 0;
+        FH_HIP(hipMemcpyAsync(&e, M->d_marchErr.p, sizeof(e), hipMemcpyDeviceToHost, M->stream));
+        FH_HIP(hipStreamSynchronize(M->stream));
+        if (e)
+        {
+            // halo slots of the pass that expired may hold stale values
+            M->march64.haloReady = M->march32.haloReady = false;
+            FH_HIP(hipMemsetAsync(M->d_marchErr.p, 0, sizeof(e), M->stream));
+            FH_HIP(hipStreamSynchronize(M->stream));
+            fail(FH_ERR_SCHEDULE, "a sweep dependency wait expired");
+        }
+    }
     if (!M->rowSweep) return;
     unsigned int e = 0;
     FH_HIP(hipMemcpyAsync(&e, M->d_rowErr.p, sizeof(e), hipMemcpyDeviceToHost, M->stream));
@@ -1823,7 +1878,7 @@ static void profile_t(fh_matrix* M, int kernel, int precon, int reps, double* ms
                 }
                 if (box && !local)
                 {
-                    box_precond_pass<T>(M, bwd, d, bwd ? part : nullptr, nullptr);
+                    box_precond_pass<T>(M, which, bwd, d, bwd ? part : nullptr, nullptr);
                     break;
                 }
                 sweep_t<T>(M, bwd ? SWEEP_PRECOND_BWD : SWEEP_PRECOND_FWD, d, nullptr, local);

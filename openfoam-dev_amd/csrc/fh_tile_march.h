@@ -1,0 +1,46 @@
+// Marching global DIC / DILU sweeps for hex boxes (fh_tile_march.hip).
+#pragma once
+
+#include "fh_tile_sweep.h"
+
+namespace fh
+{
+
+// buffers of the marching sweeps of one matrix in one precision: the pass
+// coefficients premultiplied by rD in the order the wavefronts read them,
+// and the pencil halos (every value the sentinel between launches)
+template<class T>
+struct MarchBufs
+{
+    DBuf<T> fwd, bwd, halo;
+    int kind = -1;             // factor the coefficients were packed with
+    bool haloReady = false;
+};
+
+// Boxes the marching sweeps take: below 16 planes along k the padding of
+// the skewed coefficient order (21 steps per pencil) exceeds the cells
+// themselves; a vector with 64 planes beyond each end, and a pencil's halo
+// beyond the out-of-range mark, are within 32-bit byte offsets.
+constexpr int32_t kMarchMinNz = 16;
+inline bool march_fits(int32_t nx, int32_t ny, int32_t nz, int64_t valueBytes)
+{
+    return nz >= kMarchMinNz && nz <= (1 << 18)
+           && valueBytes*nx*ny*((int64_t)nz + 128) <= 0xE0000000ll;
+}
+
+// packs dir (k, j, i coefficients of the pass, read at the neighbour with
+// dirShift) times rD for the forward or backward pass
+template<class T>
+void launch_march_pack(bool backward, const TileView& G, const T* rD, const T* const dir[3],
+                       bool dirShift, MarchBufs<T>& b, hipStream_t s);
+template<class T>
+void march_prepare_halo(const TileView& G, MarchBufs<T>& b, hipStream_t s);
+// One global DIC / DILU pass; backward with d.dotR also sums w*dotR into
+// one partial per pencil.  Returns the pencil count.
+template<class T>
+int32_t launch_sweep_march(bool backward, const TileView& G, const SweepData<T>& d,
+                           const MarchBufs<T>& b, TileSync& sync, unsigned int* err,
+                           DevState* st, hipStream_t s,
+                           const FusedFinalize& F = FusedFinalize());
+
+} // namespace fh
