@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <type_traits>
+#include <utility>
 
 
 namespace fh
@@ -1023,6 +1024,266 @@ void k_tile_dic_lds(TileView G, const float* x, const float* __restrict__ rD,
     }
 }
 
+// lane j -/+ 1 of the 16-lane row, 0 past its end
+__device__ __forceinline__ float tl_dpp_lower0(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x111, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float tl_dpp_upper0(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x101, 0xf, 0xf, true));
+}
+// the previous / next 16-lane row's lane in the same position; in the first
+// / last row any lane's value (it meets a zero coefficient)
+__device__ __forceinline__ float tl_rows_dn(float v)
+{
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v),
+                                                    false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(a[1], a[1], false, false);
+    return __uint_as_float((threadIdx.x >> 4) == 2 ? b[0] : a[0]);
+}
+__device__ __forceinline__ float tl_rows_up(float v)
+{
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v),
+                                                    false, false);
+    const auto c = __builtin_amdgcn_permlane32_swap(a[0], a[0], false, false);
+    return __uint_as_float((threadIdx.x >> 4) == 1 ? c[1] : a[1]);
+}
+
+typedef float tl_f4 __attribute__((ext_vector_type(4)));
+typedef unsigned int tl_u2 __attribute__((ext_vector_type(2)));
+
+// f(0) .. f(15) with constant arguments: a register array indexed by them
+// is never indexed by a variable, not even before loops are unrolled
+template<class F, int... S>
+__device__ __forceinline__ void tl_each(F&& f, std::integer_sequence<int, S...>)
+{
+    (f(std::integral_constant<int, S>{}), ...);
+}
+template<class F>
+__device__ __forceinline__ void tl_each16(F&& f)
+{
+    tl_each(f, std::make_integer_sequence<int, 16>{});
+}
+
+// slots turned on by q, or back (BACK): a[s] <- a[s - q]
+template<bool BACK, class V>
+__device__ __forceinline__ void tl_turn(V (&a)[16], int q)
+{
+    auto by = [&](auto dc) {
+        constexpr int d = decltype(dc)::value;
+        const bool on = (q & d) != 0;
+        V t[16];
+        tl_each16([&](auto sc) { t[decltype(sc)::value] = a[decltype(sc)::value]; });
+        tl_each16([&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            a[s] = on ? t[(BACK ? s + d : s - d) & 15] : t[s];
+        });
+    };
+    by(std::integral_constant<int, 1>{});
+    by(std::integral_constant<int, 2>{});
+}
+
+__device__ __forceinline__ tl_f4 tl_h4(tl_u2 v)
+{
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    // (through scalars: a bit cast of a vector element reads the first one)
+    const unsigned int a = v.x, b = v.y;
+    const h2 lo = __builtin_bit_cast(h2, a), hi = __builtin_bit_cast(h2, b);
+    return tl_f4{(float)lo.x, (float)lo.y, (float)hi.x, (float)hi.y};
+}
+
+// The symmetric tile-local DIC with the whole tile in registers: one
+// wavefront per tile, 224 values per lane (r, rD and the FP16 coefficients
+// of its 16 quarter rows), every input read and w written once.
+//
+// The work of a step, its order and its arithmetic are those of
+// k_tile_dic_lds: lane (j, q) owns quarter q of the rows (j, k), forward
+// step t takes k = t - j - q and backward step t takes k = 33 - t - j - q.
+// A register array cannot be indexed by a lane's own k, so row k lies in
+// slot (k + j + q) mod 16: step t then uses slot t mod 16 (1 - t mod 16
+// backward) in every lane, known at compile time with 16 steps unrolled.
+// The loads place row k in slot (k + j) mod 16, so that the four quarters
+// of a row are one 64-byte access, and two rounds of selects turn the slots
+// on by q; the results are turned back before the stores.
+//
+// The coefficients stay FP16 in their registers (half the loads of FP32,
+// and converted where they are used: kept converted across the passes they
+// cost 40 us at 256^3), and every mask of the passes is a zero coefficient
+// set once after the loads.
+//
+// What bounds it: a step is about 50 instructions of one wavefront per SIMD
+// (the registers allow no second one), and the code is about 42 KB, fetched
+// by every CU in every launch.  Measured at 256^3 (4096 tiles): 106 us, 2.8
+// TB/s of the 302 MB it has to move, against 146 us for the row walk and 167
+// us for the staged tile (59 KB of LDS allow two tiles per CU, the registers
+// four); 32^3: 14 us against 18 staged.  Loading plane by plane (slots
+// turned by j + q, twice the selects) measured 133 us.
+template<bool DOT>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void k_tile_dic_regs(TileView G, const float* x, const float* __restrict__ rD,
+                     TlCoef<__half> C, float scale, float* w, const DevState* st,
+                     double* partials, FusedFinalize F, double* tileSum)
+{
+    if (st && st->done) return;
+    const int lane = threadIdx.x;
+    // XCD-aware order (see k_tile_dic_lds)
+    const int nT = G.nTI*G.nTJ*G.nTK;
+    const int tile = (nT & 7) == 0 ? (int)(blockIdx.x & 7)*(nT >> 3) + (int)(blockIdx.x >> 3)
+                                   : (int)blockIdx.x;
+    const int TI = tile % G.nTI, TJ = (tile/G.nTI) % G.nTJ, TK = tile/(G.nTI*G.nTJ);
+    const int ey = min(16, G.ny - TJ*16), ez = min(16, G.nz - TK*16);
+    const int64_t sy = G.nx, sz = (int64_t)G.nx*G.ny;
+    const int64_t base = TI*16 + sy*(TJ*16) + sz*(TK*16);
+    const int j = lane & 15, q = lane >> 4;
+    // rows and planes outside the mesh load the nearest ones inside it
+    const int64_t row = base + 4*q + sy*min(j, ey - 1);
+    auto at = [&](int s) -> int64_t { return row + sz*min((s - j) & 15, ez - 1); };
+    tl_f4 X[16], D[16];
+    tl_u2 K[16], J[16], I[16];
+    tl_each16([&](auto sc) { X[sc] = *reinterpret_cast<const tl_f4*>(x + at(sc)); });
+    tl_each16([&](auto sc) { K[sc] = *reinterpret_cast<const tl_u2*>(C.K + at(sc)); });
+    tl_each16([&](auto sc) { J[sc] = *reinterpret_cast<const tl_u2*>(C.J + at(sc)); });
+    tl_each16([&](auto sc) { I[sc] = *reinterpret_cast<const tl_u2*>(C.I + at(sc)); });
+    tl_each16([&](auto sc) { D[sc] = *reinterpret_cast<const tl_f4*>(rD + at(sc)); });
+    // Per cell, once: the factors of the FP16 storage, the sum of r, and
+    // zero coefficients at the tile's faces and on the rows outside the
+    // mesh, so that no neighbour value has to be masked in the passes.
+    const bool rowIn = j < ey;
+    const float inv = C.inv;
+    double dotWR = 0.0, rsum = 0.0;
+    tl_each16([&](auto sc) {
+        constexpr int s = decltype(sc)::value;
+        const int k = (s - j) & 15;
+        if constexpr (DOT)
+        {
+            const double t = (double)((X[s].x + X[s].y) + (X[s].z + X[s].w));
+            rsum += rowIn && k < ez ? t : 0.0;
+        }
+        X[s] = X[s]*scale;
+        D[s] = D[s]*inv;
+        const bool inK = k > 0 && k < ez, inJ = j > 0 && rowIn;
+        K[s] = inK ? K[s] : tl_u2{0u, 0u};
+        J[s] = inJ ? J[s] : tl_u2{0u, 0u};
+        I[s].x = q > 0 ? I[s].x : I[s].x & 0xffff0000u;
+    });
+    tl_turn<false>(X, q);
+    tl_turn<false>(K, q);
+    tl_turn<false>(J, q);
+    tl_turn<false>(I, q);
+    tl_turn<false>(D, q);
+    const int o = j + q;
+    // (the coefficients stay FP16 in their registers: converted where they
+    // are used, not kept converted across the passes)
+    auto pin = [&] {
+        tl_each16([&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            tl_u2 a = K[s], b = J[s], c = I[s];
+            asm volatile("" : "+v"(a), "+v"(b), "+v"(c));
+            K[s] = a, J[s] = b, I[s] = c;
+        });
+    };
+    // ---- forward: step t, slot t mod 16; the step before left row k of
+    // lane j - 1 and of quarter q - 1, and row k - 1, one slot back ----
+    {
+        auto step = [&](int t0, auto sc) {
+            constexpr int s = decltype(sc)::value, sp = (s + 15) & 15;
+            const bool act = rowIn && (unsigned)(t0 + s - o) < (unsigned)ez;
+            const tl_f4 po = X[sp], xr = X[s], dr = D[s];
+            const tl_f4 nj = {tl_dpp_lower0(po.x), tl_dpp_lower0(po.y), tl_dpp_lower0(po.z),
+                              tl_dpp_lower0(po.w)};
+            float prev = tl_rows_dn(po.w);
+            const tl_f4 ck = tl_h4(K[s]), cj = tl_h4(J[s]), ci = tl_h4(I[s]);
+            float dp = 0.f;
+            auto fwd = [&](float ts, float dv, float kv, float jv, float a, float b, float c) {
+                ts = __builtin_fmaf(-a, kv, ts);
+                ts = __builtin_fmaf(-b, jv, ts);
+                ts = __builtin_fmaf(-c, prev, ts);
+                const float v = dv*ts;
+                if constexpr (DOT) dp = __builtin_fmaf(v, ts, dp);
+                prev = v;
+                return v;
+            };
+            tl_f4 r;
+            r.x = fwd(xr.x, dr.x, po.x, nj.x, ck.x, cj.x, ci.x);
+            r.y = fwd(xr.y, dr.y, po.y, nj.y, ck.y, cj.y, ci.y);
+            r.z = fwd(xr.z, dr.z, po.z, nj.z, ck.z, cj.z, ci.z);
+            r.w = fwd(xr.w, dr.w, po.w, nj.w, ck.w, cj.w, ci.w);
+            X[s] = act ? r : xr;
+            if constexpr (DOT) dotWR += (double)(act ? dp : 0.f);
+        };
+#pragma unroll 1
+        for (int t0 = 0;; t0 += 16)
+        {
+            pin();
+            step(t0, std::integral_constant<int, 0>{});
+            step(t0, std::integral_constant<int, 1>{});
+            if (t0 == 32) break;
+            tl_each([&](auto u) { step(t0, std::integral_constant<int, decltype(u)::value + 2>{}); },
+                    std::make_integer_sequence<int, 14>{});
+        }
+    }
+    // ---- backward (in place): step t, slot 1 - t mod 16; everything of the
+    // step before, and the upper coefficients (the lower ones of row k + 1
+    // and of row k in the neighbour lanes), is one slot further ----
+    {
+        auto step = [&](int t0, auto uc) {
+            constexpr int u = decltype(uc)::value, s = (1 - u) & 15, sn = (2 - u) & 15;
+            const bool act = rowIn && (unsigned)(33 - t0 - u - o) < (unsigned)ez;
+            const tl_f4 po = X[sn], xr = X[s], dr = D[s];
+            const tl_f4 nj = {tl_dpp_upper0(po.x), tl_dpp_upper0(po.y), tl_dpp_upper0(po.z),
+                              tl_dpp_upper0(po.w)};
+            float next = tl_rows_up(po.x);
+            const tl_u2 jn = {__float_as_uint(tl_dpp_upper0(__uint_as_float(J[sn].x))),
+                              __float_as_uint(tl_dpp_upper0(__uint_as_float(J[sn].y)))};
+            const unsigned int in = __float_as_uint(tl_rows_up(__uint_as_float(I[sn].x)));
+            const tl_f4 ck = tl_h4(K[sn]), cj = tl_h4(jn), ci = tl_h4(I[s]);
+            const float ci4 = q < 3 ? tl_h4(tl_u2{in, 0u}).x : 0.f;
+            auto bwd = [&](float xv, float dv, float kv, float jv, float a, float b, float c) {
+                float acc = a*kv;
+                acc = __builtin_fmaf(b, jv, acc);
+                acc = __builtin_fmaf(c, next, acc);
+                const float v = __builtin_fmaf(-dv, acc, xv);
+                next = v;
+                return v;
+            };
+            tl_f4 r;
+            r.w = bwd(xr.w, dr.w, po.w, nj.w, ck.w, cj.w, ci4);
+            r.z = bwd(xr.z, dr.z, po.z, nj.z, ck.z, cj.z, ci.w);
+            r.y = bwd(xr.y, dr.y, po.y, nj.y, ck.y, cj.y, ci.z);
+            r.x = bwd(xr.x, dr.x, po.x, nj.x, ck.x, cj.x, ci.y);
+            X[s] = act ? r : xr;
+        };
+#pragma unroll 1
+        for (int t0 = 0;; t0 += 16)
+        {
+            pin();
+            step(t0, std::integral_constant<int, 0>{});
+            step(t0, std::integral_constant<int, 1>{});
+            if (t0 == 32) break;
+            tl_each([&](auto u) { step(t0, std::integral_constant<int, decltype(u)::value + 2>{}); },
+                    std::make_integer_sequence<int, 14>{});
+        }
+    }
+    tl_turn<true>(X, q);
+    tl_each16([&](auto sc) {
+        if (rowIn && ((sc - j) & 15) < ez) *reinterpret_cast<tl_f4*>(w + at(sc)) = X[sc];
+    });
+    if constexpr (DOT)
+    {
+        if (tileSum)
+        {
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) rsum += __shfl_xor(rsum, off, 64);
+            if (lane == 0) tileSum[tile] = rsum;
+        }
+        dotWR *= (double)inv;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) dotWR += __shfl_xor(dotWR, off, 64);
+        partials_arrive(dotWR, 0.0, partials, gridDim.x, blockIdx.x, F);
+    }
+}
+
 // launch with the w*r sum compiled in when partials are given
 template<int PASSES, int BZ, bool SYM, class CT>
 static void tlv_launch(dim3 grid, hipStream_t s, const TileView& G, const float* x,
@@ -1049,22 +1310,26 @@ int32_t launch_tile_local_apply_f32(const TileView& G, const float* x, const flo
     const int nTiles = G.nTI*G.nTJ*G.nTK;
     const dim3 grid((nTiles + 3)/4);
     constexpr int BZ = TileBZ<float>::pre;
-    // symmetric: the row walk (default; it reads the tile's inputs again in
-    // the backward pass), the tile staged in LDS (FOAMHIP_TILE_APPLY=lds:
-    // inputs read once, but two tiles per CU leave its latency-bound steps
-    // on one wavefront per SIMD) or the quarter-row pipeline from HBM
-    // (FOAMHIP_TILE_APPLY=quarter; its per-lane quarter rows touch four
-    // times the cache lines)
-    // (read at every launch, so a process can switch between them).  By
-    // default the staged tile up to 512 tiles (all tiles in one round at two
-    // per CU: its shorter per-tile latency wins -- a serving sample of 16^3
-    // to 128^3 boxes: 196 against 180 solves/s, p50 15 against 31 ms), the
-    // row walk above (256^3: 149 against 167 us)
+    // symmetric with FP16 coefficients: the tile in registers or staged in
+    // LDS, by the number of tiles.  The register kernel is the shorter chain
+    // for one tile and holds four tiles per CU where the staged one holds
+    // two, but its 42 KB of straight code are fetched by every CU: with up
+    // to 512 tiles (all resident at once in either) that fetch is its time.
+    // Registers / LDS, back to back: 8 tiles (32^3) 14.1 / 18.1 us, 27
+    // tiles 15.8 / 18.4, 64 tiles 18.6 / 17.6, 216 tiles 26.4 / 18.1, 512
+    // tiles (128^3) 31.1 / 21.3, 576 tiles 36.7 / 37.5, 1728 tiles (192^3)
+    // 55.7 / 76.4, 4096 tiles (256^3) 106 / 167 (the row walk 84 and 146 at
+    // the last two).  FOAMHIP_TILE_APPLY forces one: regs, lds, rows (the
+    // row walk, which reads the tile's inputs again in the backward pass)
+    // or quarter (the quarter-row pipeline from HBM, whose per-lane quarter
+    // rows touch four times the cache lines); read at every launch, so a
+    // process can switch between them.
     const char* env = std::getenv("FOAMHIP_TILE_APPLY");
     const int mode = env && std::strcmp(env, "lds") == 0 ? 0
                    : env && std::strcmp(env, "quarter") == 0 ? 1
                    : env && std::strcmp(env, "rows") == 0 ? 2
-                   : nTiles <= 512 ? 0 : 2;
+                   : env && std::strcmp(env, "regs") == 0 ? 3
+                   : nTiles > 32 && nTiles <= 512 ? 0 : 3;
     // the staged tile (FP16 coefficients): 59 KB of LDS per workgroup, taken
     // when the device allows that much
     const size_t ldsBytes = (size_t)TL_LDS_CELLS*(4 + 4) + (size_t)TL_HCELLS*3*sizeof(__half);
@@ -1075,7 +1340,19 @@ int32_t launch_tile_local_apply_f32(const TileView& G, const float* x, const flo
             return (size_t)0;
         return (size_t)v;
     }();
-    if (symmetric && half3 && BZ == 16 && mode == 0 && ldsBytes <= ldsMax)
+    if (symmetric && half3 && BZ == 16 && (mode == 3 || (mode == 0 && ldsBytes > ldsMax)))
+    {
+        const dim3 gq((unsigned)nTiles);
+        const TlCoef<__half> h{half3[0], half3[1], half3[2], 1.f/halfScale};
+        if (partials)
+            hipLaunchKernelGGL((k_tile_dic_regs<true>), gq, dim3(64), 0, s, G, x, rD, h,
+                               halfScale, w, st, partials, F, tileSum);
+        else
+            hipLaunchKernelGGL((k_tile_dic_regs<false>), gq, dim3(64), 0, s, G, x, rD, h,
+                               halfScale, w, st, partials, F, tileSum);
+        return (int32_t)gq.x;
+    }
+    if (symmetric && half3 && BZ == 16 && mode == 0)
     {
         const dim3 gq((unsigned)nTiles);
         const TlCoef<__half> h{half3[0], half3[1], half3[2], 1.f/halfScale};

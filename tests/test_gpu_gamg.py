@@ -557,6 +557,26 @@ def test_tile_dic_apply_variants(apply, shape, monkeypatch):
     assert np.abs(b - om.Amul(psi)).sum() / perf.normFactor < 1e-8
 
 
+@pytest.mark.parametrize("shape", [(16, 16, 16), (16, 17, 15), (32, 1, 3), (48, 40, 37),
+                                   (37, 40, 21), (144, 130, 113)])
+def test_tile_dic_in_registers(shape, monkeypatch):
+    """The symmetric tile-local DIC with the tile in registers: one tile, one
+    row or plane of a tile, partial tiles in every direction, and more tiles
+    than stay resident at once.  Its operations and their order are those of
+    the tile staged in LDS, so the results are the same bits."""
+    nx, ny, nz = shape
+    n, lower, upper = box(nx, ny, nz)
+    rng = np.random.default_rng(29)
+    diag, up = spd_coeffs(n, lower, upper, rng)
+    m = fh.lduMatrix(fh.lduAddressing(n, lower, upper), diag, up)
+    r = rng.standard_normal(n)
+    monkeypatch.setenv("FOAMHIP_TILE_APPLY", "lds")
+    w_lds = m.precondition_f32("tileDIC", r)
+    monkeypatch.setenv("FOAMHIP_TILE_APPLY", "regs")
+    w = m.precondition_f32("tileDIC", r)
+    assert np.array_equal(w, w_lds)
+
+
 AGG_CASES = [
     ("box", lambda r: box(19, 14, 11), "spd", 1),
     ("box_merge2", lambda r: box(24, 20, 9), "spd", 2),
