@@ -50,11 +50,13 @@ struct Resident
 
 // device bytes of one resident matrix with its solver work space: FP64 and
 // FP32 row values, face-ordered coefficients, packed FP32 tile
-// coefficients, factors and about twenty work vectors
+// coefficients, factors and about twenty work vectors, and on a box the
+// buffers of the marching sweeps
 int64_t footprint_of(const fh_mesh* m)
 {
     const int64_t N = m->nCells, F = m->nFaces, nnz = m->nnzPad;
-    return 12*(N + nnz) + 16*F + 24*N + 40*N + 8*20*N + 4*12*N + (1 << 20);
+    return 12*(N + nnz) + 16*F + 24*N + 40*N + 8*20*N + 4*12*N + (1 << 20)
+           + (m->tiled ? fh::march_bytes(m->boxNx, m->boxNy, m->boxNz) : 0);
 }
 
 } // namespace

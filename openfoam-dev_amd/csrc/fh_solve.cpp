@@ -184,6 +184,7 @@ void matrix_coeffs_updated(fh_matrix* M)
     M->halfState = 0;
     M->coarseState = 0;
     M->march64.kind = M->march32.kind = -1;
+    M->march64.gsFwdReady = M->march64.gsBwdReady = false;
     for (int i = 0; i < 5; i++) M->rDValid[i] = M->rD32Valid[i] = false;
     gamg_invalidate(M);
 }
@@ -552,6 +553,16 @@ template<> void sweep_t<float>(fh_matrix* M, int kind, const SweepData<float>& d
     sweep_f(M, kind, d, st, local);
 }
 
+// FOAMHIP_BOX_SWEEP: 0 default, 1 wide, 2 wave
+static int box_sweep_forced()
+{
+    static const int forced = [] {
+        const char* e = std::getenv("FOAMHIP_BOX_SWEEP");
+        return !e ? 0 : std::strcmp(e, "wide") == 0 ? 1 : std::strcmp(e, "wave") == 0 ? 2 : 0;
+    }();
+    return forced;
+}
+
 template<class T> static MarchBufs<T>& march_bufs(fh_matrix* M);
 template<> MarchBufs<double>& march_bufs<double>(fh_matrix* M) { return M->march64; }
 template<> MarchBufs<float>& march_bufs<float>(fh_matrix* M) { return M->march32; }
@@ -594,10 +605,7 @@ static int32_t box_precond_pass(fh_matrix* M, int which, bool backward, const Sw
         d.dotR = d.x;
         d.partials = partials;
     }
-    static const int forced = [] {
-        const char* e = std::getenv("FOAMHIP_BOX_SWEEP");
-        return !e ? 0 : std::strcmp(e, "wide") == 0 ? 1 : std::strcmp(e, "wave") == 0 ? 2 : 0;
-    }();
+    const int forced = box_sweep_forced();
     if (forced != 1)
     {
         TileSync ts = M->tile_sync();
@@ -624,6 +632,36 @@ static int32_t box_precond_pass(fh_matrix* M, int which, bool backward, const Sw
     sweep_t<T>(M, backward ? SWEEP_PRECOND_BWD : SWEEP_PRECOND_FWD, d, st, false);
     const TileView G = M->tile_view(pre_bz<T>(M));
     return G.nTI*G.nTJ*G.nTK;
+}
+
+// One FP64 Gauss-Seidel sweep of d.w with source d.x: marching pencils on a
+// box with planes enough, else the general dispatch.
+static void gs_pass(fh_matrix* M, bool backward, const SweepData<double>& d0, DevState* st)
+{
+    const fh_mesh* mesh = M->mesh;
+    if (!mesh->tiled || box_sweep_forced() != 0
+        || !march_fits(mesh->boxNx, mesh->boxNy, mesh->boxNz, sizeof(double)))
+    {
+        sweep_t<double>(M, backward ? SWEEP_GS_BWD : SWEEP_GS_FWD, d0, st);
+        return;
+    }
+    MarchBufs<double>& b = M->march64;
+    const TileView G = M->tile_view(16, 8);
+    bool& ready = backward ? b.gsBwdReady : b.gsFwdReady;
+    if (!ready)
+    {
+        SweepData<double> c{};
+        set_sweep_dirs<double>(M, c, backward);
+        launch_march_pack_gs(backward, G, d0.diag, c.dir, c.dirShift != 0, b, M->stream);
+        ready = true;
+    }
+    march_prepare_halo<double>(G, b, M->stream);
+    SweepData<double> d = d0;
+    set_sweep_dirs<double>(M, d, !backward);       // the other side
+    TileSync ts = M->tile_sync();
+    launch_sweep_march_gs(backward, G, d, b, ts, M->d_marchErr.p, st, M->stream);
+    M->tileTicketBase = ts.ticketBase;
+    M->tileEpoch = ts.epoch;
 }
 
 template<class T>
@@ -1171,16 +1209,16 @@ void smooth_t(fh_matrix* M, int smoother, T* psi, const T* src, int32_t nSweeps,
                 for (int32_t s = 0; s < nSweeps; s++)
                 {
                     launch_interface_bprime(M->rows(), val, psi, src, wk[1].p, M->stream);
-                    sweep_t<T>(M, SWEEP_GS_FWD, d, st);
-                    if (sym) sweep_t<T>(M, SWEEP_GS_BWD, d, st);
+                    gs_pass(M, false, d, st);
+                    if (sym) gs_pass(M, true, d, st);
                 }
                 return;
             }
-        }
-        for (int32_t s = 0; s < nSweeps; s++)
-        {
-            sweep_t<T>(M, SWEEP_GS_FWD, d, st);
-            if (sym) sweep_t<T>(M, SWEEP_GS_BWD, d, st);
+            for (int32_t s = 0; s < nSweeps; s++)
+            {
+                gs_pass(M, false, d, st);
+                if (sym) gs_pass(M, true, d, st);
+            }
         }
     };
     auto ilu = [&](bool dilu)

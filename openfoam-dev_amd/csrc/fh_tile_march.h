@@ -1,4 +1,5 @@
-// Marching global DIC / DILU sweeps for hex boxes (fh_tile_march.hip).
+// Marching global DIC / DILU and Gauss-Seidel sweeps for hex boxes
+// (fh_tile_march.hip).
 #pragma once
 
 #include "fh_tile_sweep.h"
@@ -15,6 +16,11 @@ struct MarchBufs
     DBuf<T> fwd, bwd, halo;
     int kind = -1;             // factor the coefficients were packed with
     bool haloReady = false;
+    // Gauss-Seidel: coefficients and diagonal of the two passes, products of
+    // the old values (forward) and the source less the lower products
+    // (backward) of the running sweep
+    DBuf<T> gsFwd, gsBwd, gsOld, gsPrime;
+    bool gsFwdReady = false, gsBwdReady = false;
 };
 
 // Boxes the marching sweeps take: below 16 planes along k the padding of
@@ -28,11 +34,24 @@ inline bool march_fits(int32_t nx, int32_t ny, int32_t nz, int64_t valueBytes)
            && valueBytes*nx*ny*((int64_t)nz + 128) <= 0xE0000000ll;
 }
 
+// device bytes of all these buffers in FP64 (7 values per cell for DIC or
+// DILU, 11 and one unpadded for Gauss-Seidel, the halos)
+inline int64_t march_bytes(int32_t nx, int32_t ny, int32_t nz)
+{
+    if (!march_fits(nx, ny, nz, 8)) return 0;
+    const int64_t col = (int64_t)((nx + 15)/16)*((ny + 15)/16)*16;
+    return 8*(18*col*16*(nz + 36) + (int64_t)nx*ny*nz + 2*col*(nz + 16));
+}
+
 // packs dir (k, j, i coefficients of the pass, read at the neighbour with
 // dirShift) times rD for the forward or backward pass
 template<class T>
 void launch_march_pack(bool backward, const TileView& G, const T* rD, const T* const dir[3],
                        bool dirShift, MarchBufs<T>& b, hipStream_t s);
+// the same for the Gauss-Seidel rows, with the diagonal
+void launch_march_pack_gs(bool backward, const TileView& G, const double* diag,
+                          const double* const dir[3], bool dirShift, MarchBufs<double>& b,
+                          hipStream_t s);
 template<class T>
 void march_prepare_halo(const TileView& G, MarchBufs<T>& b, hipStream_t s);
 // One global DIC / DILU pass; backward with d.dotR also sums w*dotR into
@@ -42,5 +61,12 @@ int32_t launch_sweep_march(bool backward, const TileView& G, const SweepData<T>&
                            const MarchBufs<T>& b, TileSync& sync, unsigned int* err,
                            DevState* st, hipStream_t s,
                            const FusedFinalize& F = FusedFinalize());
+
+// One Gauss-Seidel sweep of d.w in place with source d.x; d.dir: the upper
+// coefficients (k, j, i) forward, the lower ones backward (the other side of
+// the sweep).  Forward reads d.w before, backward after the forward sweep.
+void launch_sweep_march_gs(bool backward, const TileView& G, const SweepData<double>& d,
+                           MarchBufs<double>& b, TileSync& sync, unsigned int* err,
+                           DevState* st, hipStream_t s);
 
 } // namespace fh

@@ -1,8 +1,10 @@
-// Marching DIC / DILU sweeps for hex boxes (the global preconditioner
-// passes of the FP64 and FP32 Krylov solvers).
+// Marching DIC / DILU and Gauss-Seidel sweeps for hex boxes (the global
+// preconditioner passes of the FP64 and FP32 Krylov solvers, the FP64
+// Gauss-Seidel smoothers).
 //
 // The recurrences are those of fh_tile_sweep.hip (DICPreconditioner.C:
-// 87-123, DILUPreconditioner.C:88-135): cell (i,j,k) waits for its lower
+// 87-123, DILUPreconditioner.C:88-135, GaussSeidelSmoother.C:66-187,
+// symGaussSeidelSmoother.C:66-216): cell (i,j,k) waits for its lower
 // neighbours (forward) or upper neighbours (backward, the same in reversed
 // coordinates), and each row keeps the reference face order (k, j, i), so
 // the results are bitwise those of the sequential loops.
@@ -44,6 +46,21 @@
 //     128^3            152 / 163   288 / 302   121 / 131   286 / 307
 //     200 x 150 x 133  208 / 222   382 / 394   180 / 191   379 / 401
 //     256^3            493 / 520   641 / 652   342 / 375   604 / 640
+// A Gauss-Seidel row also takes the values on its other side, which the
+// sweep does not change before the row is reached (forward: old ones) or at
+// all (backward: the forward pass's).  Forward their three products are
+// formed ahead in the packed order (the row subtracts them one by one after
+// the new values' products), backward the source less the lower products
+// is formed ahead as one vector, so a step reads streams only.  Against the
+// 16 x 16 x 4 tiles (us per sweep, everything included, forward /
+// forward and backward, with the residual of a solver iteration):
+//                      here          tiles
+//     16^3             33 / 53       77 / 145
+//     64^3             113 / 190     386 / 758
+//     150 x 100 x 60   213 / 405     532 / 1032
+//     256 x 256 x 16   393 / 657     611 / 1188
+//     200 x 150 x 133  565 / 878     1035 / 1955
+//     256^3            1390 / 2035   2435 / 4350
 // A step takes 0.10 (FP32) to 0.16 us (FP64) in a pencil alone, where a
 // compute unit moves 60 to 80 GB/s; a pencil starts about 20 (i) or 47 (j)
 // steps and one hand-off through memory after the one before.
@@ -113,11 +130,29 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t m_rsrc(const void* p, unsigned
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
 }
 
+// what a launch computes
+enum
+{
+    MARCH_FWD = 0,         // forward DIC / DILU pass
+    MARCH_BWD = 1,         // backward
+    MARCH_GS_FWD = 2,      // Gauss-Seidel rows ascending
+    MARCH_GS_BWD = 3       // Gauss-Seidel rows descending (symmetric)
+};
+template<int MODE> struct MarchMode
+{
+    static constexpr bool bwd = (MODE & 1) != 0, gs = MODE >= MARCH_GS_FWD;
+    static constexpr int na = MODE == MARCH_BWD ? 3 : 4;       // packed coefficients per cell
+    static constexpr int no = MODE == MARCH_GS_FWD ? 3 : 0;    // and products of old values
+    // coefficient blocks in flight (what the registers hold)
+    static constexpr int md = MODE == MARCH_GS_FWD ? 2 : MD;
+};
+
 template<class T>
 struct MarchArgs
 {
     int32_t nx, ny, nz, nPI, nPJ, nPB, nB;
     const T* coef;
+    const T* old;          // Gauss-Seidel forward: upper coefficients times old values
     const T* x;
     T* w;
     const T* dotR;
@@ -193,21 +228,26 @@ __device__ __forceinline__ void m_wait(const int* p, int need, MarchShared<T>& S
     asm volatile("" ::: "memory");
 }
 
-template<class T, bool BWD>
+template<class T, int MODE>
 __device__ __forceinline__ void march_compute(const MarchArgs<T>& A, MarchShared<T>& S,
                                               int pencil, int v, int lane, DevState* st)
 {
     typedef typename MBits<T>::V2 V2;
-    constexpr int NA = BWD ? 3 : 4;
+    constexpr int NA = MarchMode<MODE>::na, NO = MarchMode<MODE>::no, MD = MarchMode<MODE>::md;
     const int il = lane & 15, jl = lane >> 4;
     const V2* cp = reinterpret_cast<const V2*>(A.coef)
                    + (int64_t)(pencil*MW + v)*A.nB*(2*NA*64) + lane;
+    const V2* op = reinterpret_cast<const V2*>(A.old)
+                   + (int64_t)(pencil*MW + v)*A.nB*(2*NO*64) + lane;
     V2 cb[MD][2][NA];
+    V2 ob[MD][2][NO > 0 ? NO : 1];
 #pragma unroll
     for (int u = 0; u < MD; u++)
     {
 #pragma unroll
         for (int q = 0; q < 2*NA; q++) cb[u][q/NA][q % NA] = cp[(u*2*NA + q)*64];
+#pragma unroll
+        for (int q = 0; q < 2*NO; q++) ob[u][q/(NO ? NO : 1)][q % (NO ? NO : 1)] = op[(u*2*NO + q)*64];
         asm volatile("" ::: "memory");      // in the loop's order
     }
     // The j-1 value of step s: two steps back in the row before (16 lanes
@@ -231,7 +271,7 @@ __device__ __forceinline__ void march_compute(const MarchArgs<T>& A, MarchShared
     T nA = own[0], nJ = *atJ(0), nH = hcol[0];
     for (int b0 = 0; b0 < A.nB; b0 += MD)
     {
-        // the rings' rows of these 16 steps and of the next 16
+        // the rings' rows of these MD blocks of steps and of the next ones
         T* const o0 = own + ((b0*MG) & (MRS - 1))*64;
         const T* const h0 = hcol + ((b0*MG) & (MRS - 1))*MC;
         const T* const o1 = own + (((b0 + MD)*MG) & (MRS - 1))*64;
@@ -275,10 +315,35 @@ __device__ __forceinline__ void march_compute(const MarchArgs<T>& A, MarchShared
                 const T vI = m_shr(prev, hI);
                 const V2* c = cb[u][g >> 1];
                 auto comp = [&](const V2& t) { return (g & 1) ? t.y : t.x; };
-                T w = BWD ? a : comp(c[0])*a;
-                w = w - comp(c[NA - 3])*prev;
-                w = w - comp(c[NA - 2])*vJ;
-                w = w - comp(c[NA - 1])*vI;
+                T w;
+                if constexpr (MODE == MARCH_GS_FWD)
+                {
+                    // lower products k, j, i of new values, then the upper
+                    // ones i, j, k of old values
+                    const V2* o = ob[u][g >> 1];
+                    w = a - comp(c[0])*prev;
+                    w = w - comp(c[1])*vJ;
+                    w = w - comp(c[2])*vI;
+                    w = w - comp(o[0]);
+                    w = w - comp(o[1]);
+                    w = w - comp(o[2]);
+                    w = w/comp(c[3]);
+                }
+                else if constexpr (MODE == MARCH_GS_BWD)
+                {
+                    // a: the source less the lower products; upper ones i, j, k
+                    w = a - comp(c[2])*vI;
+                    w = w - comp(c[1])*vJ;
+                    w = w - comp(c[0])*prev;
+                    w = w/comp(c[3]);
+                }
+                else
+                {
+                    w = MODE == MARCH_BWD ? a : comp(c[0])*a;
+                    w = w - comp(c[NA - 3])*prev;
+                    w = w - comp(c[NA - 2])*vJ;
+                    w = w - comp(c[NA - 1])*vI;
+                }
                 o0[q*64] = w;
                 prev = w;
                 if (g == MG - 1)
@@ -293,6 +358,12 @@ __device__ __forceinline__ void march_compute(const MarchArgs<T>& A, MarchShared
                     const V2* cn = cp + (int64_t)min(b + MD, A.nB - 1)*(2*NA*64);
 #pragma unroll
                     for (int e = 0; e < 2*NA; e++) cb[u][e/NA][e % NA] = cn[e*64];
+                    if constexpr (NO > 0)
+                    {
+                        const V2* on = op + (int64_t)min(b + MD, A.nB - 1)*(2*NO*64);
+#pragma unroll
+                        for (int e = 0; e < 2*NO; e++) ob[u][e/NO][e % NO] = on[e*64];
+                    }
                     asm volatile("" ::: "memory");
                     if (!ready && b + 1 < A.nB)
                     {
@@ -311,18 +382,19 @@ __device__ __forceinline__ void march_compute(const MarchArgs<T>& A, MarchShared
 // halos of the pencils upstream, and (backward) the sum of w*dotR over the
 // finished planes.  Offsets run on by one addition; what lies outside the
 // box lies outside the buffer (a negative offset wraps there) and reads 0.
-template<class T, bool BWD>
+template<class T, int MODE>
 __device__ __forceinline__ double march_input(const MarchArgs<T>& A, MarchShared<T>& S,
                                               int pencil, int v, int lane, int nAct,
                                               DevState* st)
 {
     typedef typename MBits<T>::U U;
     typedef MBits<T> M;
+    constexpr bool BWD = MarchMode<MODE>::bwd, DOT = MODE == MARCH_BWD;
     constexpr U SENT = M::sent;
     constexpr unsigned int sT = sizeof(T);
     // input and halo blocks in flight (what the registers hold; MLAG is a
     // multiple of it where the sum is taken)
-    constexpr int MH = BWD ? 3 : 6;
+    constexpr int MH = DOT ? 3 : 6;
     constexpr unsigned int HB = MG*MC*sT;       // a halo block
     const int PI = pencil % A.nPI, PJ = pencil/A.nPI;
     const int il = lane & 15, jl = lane >> 4;
@@ -334,7 +406,7 @@ __device__ __forceinline__ double march_input(const MarchArgs<T>& A, MarchShared
     const unsigned int cxy = col ? plane0 + (BWD ? sz - 1 - (i + A.nx*j) : i + A.nx*j)*sT : M_OOB;
     const unsigned int dxy = col ? step : 0u;
     const unsigned int bytes = szB*(unsigned int)A.nz;
-    const bool dot = BWD && A.dotR != nullptr;
+    const bool dot = DOT && A.dotR != nullptr;
     const __amdgpu_buffer_rsrc_t rX = m_rsrc(A.x, bytes);
     const __amdgpu_buffer_rsrc_t rR = m_rsrc(dot ? A.dotR : A.x, dot ? bytes : 0);
     // this pencil's halo slots, by the step that reads them: i halo 4 steps
@@ -354,7 +426,7 @@ __device__ __forceinline__ double march_input(const MarchArgs<T>& A, MarchShared
     char* const ringJ = (char*)&S.haloJ[0][il];
     constexpr unsigned int RM = MRS*64*sT - 1, HM = MRS*MC*sT - 1;
     unsigned int tX = (il + 2*jl)*64*sT, tI = hk*MC*sT, tJ = jl*MC*sT;
-    U xr[MH][MG], rr[BWD ? MH : 1][MG];
+    U xr[MH][MG], rr[DOT ? MH : 1][MG];
     U hI[MH], hJ[MH], sI = SENT, sJ = SENT;
     // (dotR runs MLAG blocks behind: it starts before the first plane)
     unsigned int vX = cxy, vR = cxy - MG*MLAG*dxy;
@@ -383,7 +455,7 @@ __device__ __forceinline__ double march_input(const MarchArgs<T>& A, MarchShared
 #pragma unroll
     for (int u = 0; u < MH; u++)
     {
-        if constexpr (BWD) loadR(rr[u]);
+        if constexpr (DOT) loadR(rr[u]);
         asm volatile("" ::: "memory");
         M::template store<M_COH>(rI, 0, M_OOB, 0);
         M::template store<M_COH>(rJ, 0, M_OOB + 8, 0);
@@ -408,7 +480,7 @@ __device__ __forceinline__ double march_input(const MarchArgs<T>& A, MarchShared
             const int needC = MG*min(B - 5, A.nB), needO = MG*min(B - 9, A.nB);
             const int needN = MG*min(B - 11, A.nB);
             const int seenO = m_ld(&S.oStep[v]), seenN = m_ld(next);
-            if constexpr (BWD)
+            if constexpr (DOT)
             {
                 const int seenC = m_ld(&S.cStep[v]);
                 asm volatile("" ::: "memory");
@@ -548,7 +620,7 @@ __device__ __forceinline__ void march_output(const MarchArgs<T>& A, MarchShared<
     }
 }
 
-template<class T, bool BWD>
+template<class T, int MODE>
 __global__ __launch_bounds__(3*MW*64)
 void k_sweep_march(MarchArgs<T> A, DevState* st, FusedFinalize F)
 {
@@ -601,19 +673,19 @@ void k_sweep_march(MarchArgs<T> A, DevState* st, FusedFinalize F)
         if (role == 0)
         {
             __builtin_amdgcn_s_setprio(3);
-            march_compute<T, BWD>(A, S, pencil, v, lane, st);
+            march_compute<T, MODE>(A, S, pencil, v, lane, st);
             __builtin_amdgcn_s_setprio(0);
         }
         else if (role == 1)
         {
             __builtin_amdgcn_s_setprio(2);
-            march_output<T, BWD>(A, S, pencil, v, lane, st);
+            march_output<T, MarchMode<MODE>::bwd>(A, S, pencil, v, lane, st);
             __builtin_amdgcn_s_setprio(0);
         }
         else
         {
-            double acc = march_input<T, BWD>(A, S, pencil, v, lane, nAct, st);
-            if constexpr (BWD)
+            double acc = march_input<T, MODE>(A, S, pencil, v, lane, nAct, st);
+            if constexpr (MODE == MARCH_BWD)
             {
 #pragma unroll
                 for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
@@ -621,7 +693,7 @@ void k_sweep_march(MarchArgs<T> A, DevState* st, FusedFinalize F)
             }
         }
     }
-    if constexpr (BWD)
+    if constexpr (MODE == MARCH_BWD)
     {
         if (A.dotR == nullptr) return;
         __syncthreads();
@@ -632,48 +704,94 @@ void k_sweep_march(MarchArgs<T> A, DevState* st, FusedFinalize F)
     }
 }
 
-// Coefficients of one pass in wavefront order: for wavefront (pencil, v),
-// block of 4 steps, pair of steps and coefficient q, lane's two values.
-template<class T, bool BWD>
-__global__ __launch_bounds__(64)
-void k_march_pack(int nx, int ny, int nz, int nPI, int nB, const T* rD, const T* dK, const T* dJ,
-                  const T* dI, int shift, typename MBits<T>::V2* out)
+// Values of one pass in wavefront order: for wavefront (pencil, v), block of
+// 4 steps, pair of steps and value q, lane's two values.  DIC / DILU passes:
+// rD (forward) and the three coefficients times it; Gauss-Seidel: the
+// coefficients and the diagonal (rD); OLD: the coefficients times rD (psi)
+// at the neighbour on the other side.
+// A workgroup writes one value of 64 steps of one wavefront: it reads the planes these steps touch as rows of 16 cells and turns them
+// into steps in LDS.  (Read in step order every lane is in another plane:
+// with that the products of a 256^3 forward sweep took longer than the
+// sweep.)
+constexpr int MPS = 64;           // steps per workgroup
+template<class T, int MODE, bool OLD>
+__global__ __launch_bounds__(256)
+void k_march_pack(int nx, int ny, int nz, int nPI, int nB, const T* __restrict__ rD,
+                  const T* __restrict__ dK, const T* __restrict__ dJ, const T* __restrict__ dI,
+                  int shift, typename MBits<T>::V2* __restrict__ out, const DevState* st)
 {
     typedef typename MBits<T>::V2 V2;
-    constexpr int NA = BWD ? 3 : 4;
-    const int wv = blockIdx.x, pencil = wv/MW, v = wv % MW, lane = threadIdx.x;
+    constexpr bool BWD = MarchMode<MODE>::bwd, GS = MarchMode<MODE>::gs;
+    constexpr int NA = OLD ? MarchMode<MODE>::no : MarchMode<MODE>::na;
+    __shared__ T buf[MPS][64];
+    if (st && st->done) return;
+    const int wv = blockIdx.x, pencil = wv/MW, v = wv % MW;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int PI = pencil % nPI, PJ = pencil/nPI;
     const int il = lane & 15, jl = lane >> 4;
     const int i = PI*MC + il, j = PJ*MC + MW*v + jl;
     if (PJ*MC + MW*v >= ny) return;
     const bool col = i < nx && j < ny;
     const int64_t sy = nx, sz = (int64_t)nx*ny, last = sz*nz - 1;
-    const int64_t off[3] = {shift ? sz : 0, shift ? sy : 0, shift ? 1 : 0};
-    const T* dir[3] = {dK, dJ, dI};
-    const int b1 = min(nB, (int)(blockIdx.y + 1)*MD);
-    for (int b = blockIdx.y*MD; b < b1; b++)
-#pragma unroll
-        for (int p = 0; p < 2; p++)
+    const int s0 = blockIdx.y*MPS, s1 = min(s0 + MPS, nB*MG);
+    // value q: the product or coefficient of direction e (k, j, i), or the
+    // factor itself
+    const int q = blockIdx.z;
+    const int e = OLD ? 2 - q : GS ? q : q - (NA - 3);
+    const bool factor = e < 0 || e > 2;
+    const T* const dir = e == 2 ? dI : e == 1 ? dJ : dK;
+    const int64_t off = e == 2 ? 1 : e == 1 ? sy : sz;
+    const bool inPlane = OLD ? (e == 2 ? i < nx - 1 : e == 1 ? j < ny - 1 : true)
+                             : (e == 2 ? i > 0 : e == 1 ? j > 0 : true);
+    const bool use = col && (factor || inPlane);
+    const int kLo = !OLD && e == 0 ? 1 : 0, kHi = OLD && e == 0 ? nz - 1 : nz;
+#pragma unroll 8
+    for (int k = s0 - MSKEW + wave; k < s1; k += 4)
+    {
+        const bool ok = use && k >= kLo && k < kHi;
+        const int64_t cf = ok ? i + sy*j + sz*k : 0;
+        const int64_t c = BWD ? last - cf : cf;
+        T t;
+        if (factor) t = ok ? rD[c] : T(GS ? 1 : 0);
+        else
         {
-            T t[2][NA];
-#pragma unroll
-            for (int h = 0; h < 2; h++)
-            {
-                const int k = MG*b + 2*p + h - il - 2*jl;
-                const bool ok = col && k >= 0 && k < nz;
-                const int64_t cf = ok ? i + sy*j + sz*k : 0;
-                const int64_t c = BWD ? last - cf : cf;
-                const bool has[3] = {ok && k > 0, ok && j > 0, ok && i > 0};
-                const T r = ok ? rD[c] : T(0);
-                if constexpr (!BWD) t[h][0] = r;
-#pragma unroll
-                for (int e = 0; e < 3; e++)
-                    t[h][NA - 3 + e] = has[e] ? r*dir[e][c + off[e]] : T(0);
-            }
-            V2* o = out + (((int64_t)wv*nB + b)*2 + p)*NA*64 + lane;
-#pragma unroll
-            for (int q = 0; q < NA; q++) o[q*64] = V2{t[0][q], t[1][q]};
+            const T a = dir[ok && shift ? c + off : c];
+            if constexpr (OLD) t = a*rD[ok ? c + off : c];
+            else if constexpr (GS) t = a;
+            else t = rD[c]*a;
+            t = ok ? t : T(0);
         }
+        const int s = k + il + 2*jl - s0;
+        if (s >= 0 && s < MPS) buf[s][lane] = t;
+    }
+    __syncthreads();
+    for (int h = wave; h < (s1 - s0)/2; h += 4)
+        out[((int64_t)wv*nB*2 + s0/2 + h)*NA*64 + q*64 + lane] =
+            V2{buf[2*h][lane], buf[2*h + 1][lane]};
+}
+
+// The source of the backward Gauss-Seidel rows: b less the lower products
+// k, j, i of the forward pass's values (symGaussSeidelSmoother.C:139-183)
+template<class T>
+__global__ __launch_bounds__(256)
+void k_march_prime(int nx, int ny, int nz, const T* b, const T* psi, const T* dK, const T* dJ,
+                   const T* dI, T* out, const DevState* st)
+{
+    if (st && st->done) return;
+    const int sy = nx;
+    const int64_t sz = (int64_t)nx*ny;
+    const int q = blockIdx.x*256 + threadIdx.x;
+    if (q >= sz) return;
+    const int j = q/nx, i = q - j*nx;
+    for (int k = blockIdx.y; k < nz; k += gridDim.y)
+    {
+        const int64_t c = q + sz*k;
+        T t = b[c];
+        if (k > 0) t = t - dK[c]*psi[c - sz];
+        if (j > 0) t = t - dJ[c]*psi[c - sy];
+        if (i > 0) t = t - dI[c]*psi[c - 1];
+        out[c] = t;
+    }
 }
 
 template<class U>
@@ -693,25 +811,36 @@ static void march_shape(const TileView& G, int32_t& nPI, int32_t& nPJ, int32_t& 
     nB = (nB + MD - 1)/MD*MD;
 }
 
+template<class T, int MODE, bool OLD>
+static void march_pack(const TileView& G, const T* rD, const T* const dir[3], bool dirShift,
+                       DBuf<T>& out, const DevState* st, hipStream_t s)
+{
+    int32_t nPI, nPJ, nPB, nB;
+    march_shape(G, nPI, nPJ, nPB, nB);
+    const int64_t waves = (int64_t)nPI*nPJ*MW;
+    const int nv = OLD ? MarchMode<MODE>::no : MarchMode<MODE>::na;
+    out.alloc((size_t)waves*nB*MG*64*nv);
+    hipLaunchKernelGGL((k_march_pack<T, MODE, OLD>),
+                       dim3((unsigned)waves, (unsigned)((nB*MG + MPS - 1)/MPS), (unsigned)nv),
+                       dim3(256), 0, s, G.nx, G.ny, G.nz, nPI, nB, rD, dir[0], dir[1], dir[2],
+                       dirShift ? 1 : 0, reinterpret_cast<typename MBits<T>::V2*>(out.p), st);
+}
+
 template<class T>
 void launch_march_pack(bool backward, const TileView& G, const T* rD, const T* const dir[3],
                        bool dirShift, MarchBufs<T>& b, hipStream_t s)
 {
-    typedef typename MBits<T>::V2 V2;
-    int32_t nPI, nPJ, nPB, nB;
-    march_shape(G, nPI, nPJ, nPB, nB);
-    const int64_t waves = (int64_t)nPI*nPJ*MW;
-    DBuf<T>& d = backward ? b.bwd : b.fwd;
-    d.alloc((size_t)waves*nB*MG*64*(backward ? 3 : 4));
-    const dim3 grid((unsigned)waves, (unsigned)(nB/MD));
+    if (backward) march_pack<T, MARCH_BWD, false>(G, rD, dir, dirShift, b.bwd, nullptr, s);
+    else march_pack<T, MARCH_FWD, false>(G, rD, dir, dirShift, b.fwd, nullptr, s);
+}
+
+void launch_march_pack_gs(bool backward, const TileView& G, const double* diag,
+                          const double* const dir[3], bool dirShift, MarchBufs<double>& b,
+                          hipStream_t s)
+{
     if (backward)
-        hipLaunchKernelGGL((k_march_pack<T, true>), grid, dim3(64), 0, s, G.nx, G.ny, G.nz, nPI,
-                           nB, rD, dir[0], dir[1], dir[2], dirShift ? 1 : 0,
-                           reinterpret_cast<V2*>(d.p));
-    else
-        hipLaunchKernelGGL((k_march_pack<T, false>), grid, dim3(64), 0, s, G.nx, G.ny, G.nz, nPI,
-                           nB, rD, dir[0], dir[1], dir[2], dirShift ? 1 : 0,
-                           reinterpret_cast<V2*>(d.p));
+        march_pack<double, MARCH_GS_BWD, false>(G, diag, dir, dirShift, b.gsBwd, nullptr, s);
+    else march_pack<double, MARCH_GS_FWD, false>(G, diag, dir, dirShift, b.gsFwd, nullptr, s);
 }
 
 template<class T>
@@ -730,34 +859,74 @@ void march_prepare_halo(const TileView& G, MarchBufs<T>& b, hipStream_t s)
 }
 
 template<class T>
+static MarchArgs<T> march_args(const TileView& G, const MarchBufs<T>& b, const TileSync& sync,
+                               unsigned int* err)
+{
+    if (!b.haloReady) fail(FH_ERR_INVALID, "internal: marching sweep without its halos");
+    MarchArgs<T> A{};
+    A.nx = G.nx; A.ny = G.ny; A.nz = G.nz;
+    march_shape(G, A.nPI, A.nPJ, A.nPB, A.nB);
+    A.halo = b.halo.p;
+    A.ticket = sync.ticket;
+    A.ticketBase = sync.ticketBase;
+    A.err = err;
+    return A;
+}
+
+template<class T, int MODE>
+static int32_t march_launch(const MarchArgs<T>& A, TileSync& sync, DevState* st, hipStream_t s,
+                            const FusedFinalize& F = FusedFinalize())
+{
+    const int32_t nP = A.nPI*A.nPJ;
+    hipLaunchKernelGGL((k_sweep_march<T, MODE>), dim3(nP), dim3(3*MW*64), 0, s, A, st, F);
+    sync.ticketBase += (unsigned long long)nP;
+    sync.epoch++;
+    return nP;
+}
+
+template<class T>
 int32_t launch_sweep_march(bool backward, const TileView& G, const SweepData<T>& d,
                            const MarchBufs<T>& b, TileSync& sync, unsigned int* err,
                            DevState* st, hipStream_t s, const FusedFinalize& F)
 {
-    if (!b.haloReady || !b.fwd.p || !b.bwd.p)
+    if (!b.fwd.p || !b.bwd.p)
         fail(FH_ERR_INVALID, "internal: marching sweep without its buffers");
     if (d.dotR && (!backward || !d.partials))
         fail(FH_ERR_INVALID, "internal: fused sum on a sweep that does not provide it");
-    MarchArgs<T> A;
-    A.nx = G.nx; A.ny = G.ny; A.nz = G.nz;
-    march_shape(G, A.nPI, A.nPJ, A.nPB, A.nB);
+    MarchArgs<T> A = march_args<T>(G, b, sync, err);
     A.coef = backward ? b.bwd.p : b.fwd.p;
     A.x = backward ? d.w : d.x;
     A.w = d.w;
     A.dotR = backward ? d.dotR : nullptr;
     A.partials = d.partials;
-    A.halo = b.halo.p;
-    A.ticket = sync.ticket;
-    A.ticketBase = sync.ticketBase;
-    A.err = err;
-    const int32_t nP = A.nPI*A.nPJ;
-    if (backward)
-        hipLaunchKernelGGL((k_sweep_march<T, true>), dim3(nP), dim3(3*MW*64), 0, s, A, st, F);
-    else
-        hipLaunchKernelGGL((k_sweep_march<T, false>), dim3(nP), dim3(3*MW*64), 0, s, A, st, F);
-    sync.ticketBase += (unsigned long long)nP;
-    sync.epoch++;
-    return nP;
+    return backward ? march_launch<T, MARCH_BWD>(A, sync, st, s, F)
+                    : march_launch<T, MARCH_FWD>(A, sync, st, s, F);
+}
+
+void launch_sweep_march_gs(bool backward, const TileView& G, const SweepData<double>& d,
+                           MarchBufs<double>& b, TileSync& sync, unsigned int* err,
+                           DevState* st, hipStream_t s)
+{
+    MarchArgs<double> A = march_args<double>(G, b, sync, err);
+    A.w = d.w;
+    if (!backward)
+    {
+        march_pack<double, MARCH_GS_FWD, true>(G, d.w, d.dir, d.dirShift != 0, b.gsOld, st, s);
+        A.coef = b.gsFwd.p;
+        A.old = b.gsOld.p;
+        A.x = d.x;
+        march_launch<double, MARCH_GS_FWD>(A, sync, st, s);
+        return;
+    }
+    const int64_t sz = (int64_t)G.nx*G.ny;
+    b.gsPrime.alloc((size_t)(sz*G.nz));
+    const unsigned gx = (unsigned)((sz + 255)/256);
+    const unsigned gy = (unsigned)std::max<int64_t>(1, std::min<int64_t>(G.nz, 4096/gx));
+    hipLaunchKernelGGL((k_march_prime<double>), dim3(gx, gy), dim3(256), 0, s, G.nx, G.ny, G.nz,
+                       d.x, d.w, d.dir[0], d.dir[1], d.dir[2], b.gsPrime.p, st);
+    A.coef = b.gsBwd.p;
+    A.x = b.gsPrime.p;
+    march_launch<double, MARCH_GS_BWD>(A, sync, st, s);
 }
 
 #define MARCH_INST(T) \

@@ -71,3 +71,20 @@ def test_march_solves(size, kind):
     r = rng.standard_normal(c.N)
     p = ctl["preconditioner"]
     np.testing.assert_array_equal(m.precondition(p, r), om.precondition(p, r))
+
+
+@pytest.mark.parametrize("size", SIZES)
+@pytest.mark.parametrize("kind", ["spd", "asym"])
+@pytest.mark.parametrize("smoother", ["GaussSeidel", "symGaussSeidel"])
+def test_march_gauss_seidel_bitwise(size, kind, smoother):
+    """Gauss-Seidel sweeps from a start that is not zero, two of them and one
+    more on the same matrix, and again after its coefficients changed."""
+    c, rng, m, om = systems(size, kind)
+    psi, b = rng.standard_normal(c.N), rng.standard_normal(c.N)
+    for n in (2, 1):
+        ref = om.smooth(smoother, psi, b, n)
+        np.testing.assert_array_equal(m.smooth(smoother, psi, b, n), ref)
+    co = (spd_coeffs if kind == "spd" else asym_coeffs)(c.N, c.lower, c.upper, rng)
+    m.set(*co)
+    om2 = O.Matrix(O.Addr(c.N, c.lower, c.upper), *co)
+    np.testing.assert_array_equal(m.smooth(smoother, psi, b, 1), om2.smooth(smoother, psi, b, 1))
