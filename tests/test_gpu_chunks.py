@@ -1,0 +1,41 @@
+"""The value-polling chunk sweeps on layered graphs: rows with as many
+dependencies as their slots (4, 8, 16, 32), one more, and more than the
+largest, against the oracle's sequential loops."""
+import numpy as np
+import pytest
+
+import foamhip as fh
+import oracle as O
+from meshes import asym_coeffs, spd_coeffs
+
+pytestmark = pytest.mark.gpu
+
+
+def layered(width, layers, deg, rng, spread):
+    """layers of `width` cells; every cell has deg neighbours in the layer
+    before (spread: 1 to deg of them), so the layers are the levels."""
+    pairs = []
+    for l in range(1, layers):
+        for c in range(width):
+            n = rng.integers(1, deg + 1) if spread else deg
+            for p in rng.choice(width, n, replace=False):
+                pairs.append(((l - 1) * width + p, l * width + c))
+    pairs = np.array(sorted(pairs), dtype=np.int32)
+    return width * layers, pairs[:, 0].copy(), pairs[:, 1].copy()
+
+
+@pytest.mark.parametrize("deg,spread", [(1, False), (4, False), (5, True), (8, False), (9, True),
+                                        (16, False), (17, True), (32, False), (45, True)])
+@pytest.mark.parametrize("kind", ["spd", "asym"])
+def test_chunk_sweeps_bitwise(deg, spread, kind):
+    rng = np.random.default_rng(41 + deg)
+    n, lower, upper = layered(70 if deg < 32 else 130, 7, deg, rng, spread)
+    co = (spd_coeffs if kind == "spd" else asym_coeffs)(n, lower, upper, rng)
+    m = fh.lduMatrix(fh.lduAddressing(n, lower, upper), *co)
+    om = O.Matrix(O.Addr(n, lower, upper), *co)
+    psi, b = rng.standard_normal(n), rng.standard_normal(n)
+    for smoother in ("GaussSeidel", "symGaussSeidel"):
+        np.testing.assert_array_equal(m.smooth(smoother, psi, b, 2),
+                                      om.smooth(smoother, psi, b, 2))
+    precon = "DIC" if kind == "spd" else "DILU"
+    np.testing.assert_array_equal(m.precondition(precon, b), om.precondition(precon, b))
