@@ -60,8 +60,8 @@ static fh_mesh* make_mesh(int device, int32_t n, const std::vector<int32_t>& lo,
         static const bool verbose = std::getenv("FOAMHIP_GAMG_VERBOSE") != nullptr;
         if (verbose)
             std::fprintf(stderr, "foamhip GAMG level: %d cells, %d faces, %d dependency levels, "
-                                 "%s\n", n, (int)lo.size(), m->sched.nLevels,
-                         m->chunkSweep ? "chunk sweep" : "one-workgroup level sweep");
+                                 "%d chunks\n", n, (int)lo.size(), m->sched.nLevels,
+                         m->nChunks);
     }
     catch (...)
     {

@@ -146,9 +146,9 @@ struct fh_mesh
     int32_t maxTiles = 0;
     hipStream_t setupStream = nullptr;
 
-    // chunks of the sync-free sweep (one-part meshes whose levels are wide
-    // enough): rows of one level, at most 64 per chunk
-    bool chunkSweep = false;
+    // chunks of the sync-free sweeps (one-part meshes): rows of one level, at
+    // most 64 per chunk; wideLevels: 16 rows or more per level on average
+    bool wideLevels = false;
     int32_t nChunks = 0;
     fh::DBuf<int32_t> d_chunkStart, d_fwdOff, d_fwdDeps, d_bwdOff, d_bwdDeps;
 

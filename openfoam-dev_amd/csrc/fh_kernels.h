@@ -147,6 +147,16 @@ struct RowSync
     unsigned int* err;                 // set when a wait expired
 };
 
+// LDS of the one-workgroup chunk sweep, and the rows that fit there
+constexpr int32_t kVfLdsBytes = 144*1024;
+template<class T> constexpr int32_t vf_lds_rows() { return kVfLdsBytes/(int32_t)sizeof(T); }
+// One sweep (Gauss-Seidel or DIC/DILU kinds, in place) by one workgroup;
+// false (nothing launched) for the other kinds and larger meshes
+template<class T>
+bool launch_sweep_chunks_lds(int kind, const RowsView& R, const SweepData<T>& d, int32_t nRows,
+                             const ChunkView& C, const RowSync& sync, DevState* st,
+                             hipStream_t s);
+
 // persistent workgroups (4 wavefronts each) of one chunk-sweep launch
 constexpr int32_t kRowSweepBlocks = 256;
 
@@ -207,11 +217,6 @@ template<class T>
 void launch_sweep_colour_run(const RowsView& R, const SweepData<T>& d, const int32_t* rows,
                              const int32_t* cstart, int32_t k0, int32_t k1, bool desc,
                              const DevState* st, hipStream_t s);
-// One-workgroup pipelined level sweep of a one-part mesh (Gauss-Seidel and
-// the DIC/DILU passes; fh_level_sweep.hip); false: kind or mesh not covered
-template<class T>
-bool launch_sweep_level_wg(int kind, const RowsView& R, const SchedView& S,
-                           const SweepData<T>& d, DevState* st, hipStream_t s);
 template<class T>
 void launch_sweep(int kind, const RowsView& R, const SchedView& S, SweepSync& sync,
                   const SweepData<T>& d, DevState* st, hipStream_t s);

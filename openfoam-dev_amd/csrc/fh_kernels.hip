@@ -692,12 +692,15 @@ template<class T> struct SweepSentinel;
 template<> struct SweepSentinel<double>
 {
     static constexpr long long bits = 0x7FF0DEAD5EED0001ll;
+    // (the upper half alone marks a signalling NaN)
+    __device__ static bool half(double v) { return (int)(__double_as_longlong(v) >> 32) == (int)(bits >> 32); }
     __device__ static double value() { return __longlong_as_double(bits); }
     __device__ static bool is(double v) { return __double_as_longlong(v) == bits; }
 };
 template<> struct SweepSentinel<float>
 {
     static constexpr int bits = 0x7FA05EED;
+    __device__ static bool half(float v) { return __float_as_int(v) == bits; }
     __device__ static float value() { return __int_as_float(bits); }
     __device__ static bool is(float v) { return __float_as_int(v) == bits; }
 };
@@ -708,9 +711,40 @@ template<> struct SweepSentinel<float>
 // the backward pass.  Dependency values come from wDep (with VF: polled
 // until no longer the sentinel), the others from wIn.  acc -= c*w
 // (Gauss-Seidel) or acc -= rD*c*w.
-template<class T, int KIND, bool BACKWARD, bool VF>
+// where the values of the sweep are polled: the output in memory, or a copy
+// of the whole vector in LDS (one workgroup sweeps the mesh)
+template<class T>
+struct VfGlobal
+{
+    static constexpr bool lds = false;
+    static constexpr int32_t pad = 0;          // an unused slot's index (masked)
+    T* w;
+    __device__ __forceinline__ T ld(int32_t i) const { return sw_ld<true>(&w[i]); }
+    __device__ __forceinline__ void st(int32_t i, T v) const { sw_st<true>(&w[i], v); }
+};
+template<class T>
+struct VfLds
+{
+    static constexpr bool lds = true;
+    static constexpr int32_t pad = vf_lds_rows<T>();   // holds zero
+    T* s;
+    T* w;
+    const int* gate;       // sequence number of the last chunk done by the wavefront ...
+    int gateNeed;          // ... that takes the chunk two before this one
+    __device__ __forceinline__ T ld(int32_t i) const
+    {
+        return __hip_atomic_load(&s[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __device__ __forceinline__ void st(int32_t i, T v) const
+    {
+        __hip_atomic_store(&s[i], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        w[i] = v;
+    }
+};
+
+template<class T, int KIND, bool BACKWARD, bool VF, class W>
 __device__ __forceinline__ T row_tail(const RowsView& R, const SweepData<T>& d, const T* wIn,
-                                      const T* wDep, int32_t base, int32_t nLo, int32_t kLo,
+                                      const W& wDep, int32_t base, int32_t nLo, int32_t kLo,
                                       int32_t kHi, T acc, T rDr, unsigned long long t0,
                                       unsigned long long waitTicks, bool& expired)
 {
@@ -735,7 +769,7 @@ __device__ __forceinline__ T row_tail(const RowsView& R, const SweepData<T>& d, 
             const int32_t k = desc ? kHi - 1 - b - j : kLo + b + j;
             const bool in = desc ? k >= kLo : k < kHi;
             const bool dep = BACKWARD ? k >= nLo : k < nLo;
-            w[j] = !in ? T(0) : dep ? sw_ld<true>(&wDep[col[j]]) : wIn[col[j]];
+            w[j] = !in ? T(0) : dep ? wDep.ld(col[j]) : wIn[col[j]];
         }
         if constexpr (VF)
         {
@@ -763,7 +797,7 @@ __device__ __forceinline__ T row_tail(const RowsView& R, const SweepData<T>& d, 
                     const int32_t k = desc ? kHi - 1 - b - j : kLo + b + j;
                     const bool in = desc ? k >= kLo : k < kHi;
                     const bool dep = BACKWARD ? k >= nLo : k < nLo;
-                    if (in && dep && SweepSentinel<T>::is(w[j])) w[j] = sw_ld<true>(&wDep[col[j]]);
+                    if (in && dep && SweepSentinel<T>::is(w[j])) w[j] = wDep.ld(col[j]);
                 }
             }
         }
@@ -799,7 +833,7 @@ __device__ __forceinline__ void row_finish(const RowsView& R, const SweepData<T>
         for (int k = 0; k < ROW_PREFETCH; k++)
             if (k < p.nEnt) t -= p.val[k]*p.w[k];
         bool unused = false;
-        t = row_tail<T, KIND, BACKWARD, false>(R, d, d.w, d.w, p.base, p.nLo, ROW_PREFETCH, p.nEnt, t, T(0),
+        t = row_tail<T, KIND, BACKWARD, false>(R, d, d.w, VfGlobal<T>{d.w}, p.base, p.nLo, ROW_PREFETCH, p.nEnt, t, T(0),
                                                0, 0, unused);
         sw_st<true>(&d.w[r], t/p.b);
     }
@@ -812,7 +846,7 @@ __device__ __forceinline__ void row_finish(const RowsView& R, const SweepData<T>
         for (int k = 0; k < ROW_PREFETCH; k++)
             if (k < p.nLo) w -= rDr*p.val[k]*p.w[k];
         bool unused = false;
-        w = row_tail<T, KIND, BACKWARD, false>(R, d, d.w, d.w, p.base, p.nLo, ROW_PREFETCH, p.nLo, w, rDr,
+        w = row_tail<T, KIND, BACKWARD, false>(R, d, d.w, VfGlobal<T>{d.w}, p.base, p.nLo, ROW_PREFETCH, p.nLo, w, rDr,
                                                0, 0, unused);
         sw_st<true>(&d.w[r], w);
     }
@@ -824,7 +858,7 @@ __device__ __forceinline__ void row_finish(const RowsView& R, const SweepData<T>
         // entries past the prefetched ones, down to the first upper entry
         const int32_t kEnd = p.nLo > ROW_PREFETCH ? p.nLo : ROW_PREFETCH;
         bool unused = false;
-        w = row_tail<T, KIND, BACKWARD, false>(R, d, d.w, d.w, p.base, p.nLo, kEnd, p.nEnt, w, rDr, 0, 0,
+        w = row_tail<T, KIND, BACKWARD, false>(R, d, d.w, VfGlobal<T>{d.w}, p.base, p.nLo, kEnd, p.nEnt, w, rDr, 0, 0,
                                                unused);
 #pragma unroll
         for (int k = ROW_PREFETCH - 1; k >= 0; k--)
@@ -960,24 +994,6 @@ void k_copy_rows(int32_t n, const T* __restrict__ a, T* __restrict__ b, const De
     if (i < n && !(st && st->done)) b[i] = a[i];
 }
 
-// one value: poll until written (or the wait expires)
-template<class T>
-__device__ __forceinline__ void vf_poll(const T* a, unsigned long long t0,
-                                        unsigned long long waitTicks, bool& expired)
-{
-    for (;;)
-    {
-        const T v = sw_ld<true>(a);
-        if (!SweepSentinel<T>::is(v)) return;
-        if ((unsigned long long)(wall_clock64() - t0) > waitTicks)
-        {
-            expired = true;
-            return;
-        }
-        __builtin_amdgcn_s_sleep(1);
-    }
-}
-
 // a row's dependency entries: nDep of them, in the order the row takes them
 // (backward preconditioner: descending)
 template<int KIND, bool BACKWARD>
@@ -986,9 +1002,9 @@ __device__ __forceinline__ int32_t vf_entry(int32_t nLo, int32_t nEnt, int32_t m
     return KIND == SWEEP_PRECOND_BWD ? nEnt - 1 - m : BACKWARD ? nLo + m : m;
 }
 
-template<class T, int KIND, bool BACKWARD, int M>
+template<class T, int KIND, bool BACKWARD, int M, class W>
 __device__ __forceinline__ void vf_rows(const RowsView& R, const SweepData<T>& d, const T* wIn,
-                                        T* wOut, int32_t r, bool have, int32_t nLo,
+                                        const W& wOut, int32_t r, bool have, int32_t nLo,
                                         int32_t nEnt, const RowSync& sync, DevState* st)
 {
     typedef SweepSentinel<T> S;
@@ -1007,7 +1023,7 @@ __device__ __forceinline__ void vf_rows(const RowsView& R, const SweepData<T>& d
     {
         const bool in = m < nDep;
         const int32_t e = base + (vf_entry<KIND, BACKWARD>(nLo, nEnt, m) << 6);
-        col[m] = in ? R.col[e] : 0;
+        col[m] = in ? R.col[e] : W::pad;
         val[m] = in ? d.val[e] : T(0);
     }
     T a = T(0), b = T(1);
@@ -1016,17 +1032,21 @@ __device__ __forceinline__ void vf_rows(const RowsView& R, const SweepData<T>& d
         b = GS ? d.diag[r] : d.rD[r];
         a = KIND == SWEEP_PRECOND_BWD ? wIn[r] : d.x[r];
     }
-    // the chunk's last dependency and the last one of that row (rows are
-    // numbered by level)
-    int32_t key = INT32_MIN;
-#pragma unroll
-    for (int m = 0; m < M; m++)
-        if (m < nDep) key = max(key, BACKWARD ? -col[m] : col[m]);
-    for (int off = 32; off > 0; off >>= 1) key = max(key, __shfl_xor(key, off, 64));
-    int32_t gate = INT32_MIN;
-    if (key != INT32_MIN)
+    // the chunk's last dependency and (memory) the last one of that row (rows
+    // are numbered by level)
+    const bool anyDep = __any(nDep > 0) != 0;
+    int32_t gate = INT32_MIN, kr = 0;
+    if (anyDep)
     {
-        const int32_t kr = __builtin_amdgcn_readfirstlane(BACKWARD ? -key : key);
+        int32_t key = INT32_MIN;
+#pragma unroll
+        for (int m = 0; m < M; m++)
+            if (m < nDep) key = max(key, BACKWARD ? -col[m] : col[m]);
+        for (int off = 32; off > 0; off >>= 1) key = max(key, __shfl_xor(key, off, 64));
+        kr = __builtin_amdgcn_readfirstlane(BACKWARD ? -key : key);
+    }
+    if (!W::lds && anyDep)
+    {
         const int32_t info = R.rowInfo[kr];
         const int32_t kLo = info & 0xffff, kEnt = info >> 16;
         const int32_t n = BACKWARD ? kEnt - kLo : kLo;
@@ -1061,42 +1081,83 @@ __device__ __forceinline__ void vf_rows(const RowsView& R, const SweepData<T>& d
         for (int m = 0; m < M; m++) val[m] = b*val[m];
     }
     // ---- the wait ----
-    if (gate != INT32_MIN && lane == 0)
-        vf_poll(&wOut[BACKWARD ? -gate : gate], t0, sync.waitTicks, expired);
+    auto late = [&] {
+        return (unsigned long long)(wall_clock64() - t0) > sync.waitTicks;
+    };
+    // (the clock is slow next to an LDS poll)
+    unsigned int spins = 0;
+    if constexpr (W::lds)
+    {
+        while (__hip_atomic_load(wOut.gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
+               < wOut.gateNeed)
+        {
+            if ((++spins & 255u) == 0 && late()) { expired = true; break; }
+            __builtin_amdgcn_s_sleep(1);
+        }
+    }
+    else if (gate != INT32_MIN && lane == 0)
+    {
+        while (SweepSentinel<T>::is(wOut.ld(BACKWARD ? -gate : gate)))
+        {
+            if (late()) { expired = true; break; }
+            __builtin_amdgcn_s_sleep(1);
+        }
+    }
+    if constexpr (W::lds) __builtin_amdgcn_s_setprio(3);
     T w[M];
-    if (key != INT32_MIN)
+    if (anyDep)
     {
         auto sample = [&](T (&v)[M]) {
 #pragma unroll
-            for (int m = 0; m < M; m++) v[m] = sw_ld<true>(&wOut[col[m]]);
+            for (int m = 0; m < M; m++) v[m] = wOut.ld(col[m]);
         };
         auto pending = [&](const T (&v)[M]) {
             bool p = false;
 #pragma unroll
-            for (int m = 0; m < M; m++) p |= m < nDep && S::is(v[m]);
+            for (int m = 0; m < M; m++) p |= (W::lds || m < nDep) && S::half(v[m]);
             return __any(p) != 0;
         };
-        T u[M];
-        sample(w);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_sleep(12);
-        for (;;)
+        if constexpr (W::lds)
         {
-            sample(u);
-            asm volatile("" ::: "memory");
-            if (!pending(w)) break;
+            // the last dependency in a short loop of its own, then (nearly
+            // always complete, as a chunk's values are one store) all
+            if constexpr (M > 4)
+            while (SweepSentinel<T>::half(wOut.ld(kr)))
+                if (expired || ((++spins & 255u) == 0 && late())) { expired = true; break; }
+            bool p;
+#pragma unroll 1
+            do
+            {
+                sample(w);
+                asm volatile("" ::: "memory");
+                p = pending(w);
+                if (p && (expired || ((++spins & 255u) == 0 && late())))
+                {
+                    expired = true;
+                    p = false;
+                }
+            } while (p);
+        }
+        else
+        {
+            T u[M];
             sample(w);
             asm volatile("" ::: "memory");
-            if (!pending(u))
+            __builtin_amdgcn_s_sleep(12);
+            for (;;)
             {
+                sample(u);
+                asm volatile("" ::: "memory");
+                if (!pending(w)) break;
+                sample(w);
+                asm volatile("" ::: "memory");
+                if (!pending(u))
+                {
 #pragma unroll
-                for (int m = 0; m < M; m++) w[m] = u[m];
-                break;
-            }
-            if (__any(expired || (unsigned long long)(wall_clock64() - t0) > sync.waitTicks))
-            {
-                expired = true;
-                break;
+                    for (int m = 0; m < M; m++) w[m] = u[m];
+                    break;
+                }
+                if (__any(expired || late())) { expired = true; break; }
             }
         }
     }
@@ -1105,7 +1166,7 @@ __device__ __forceinline__ void vf_rows(const RowsView& R, const SweepData<T>& d
     if (have)
     {
 #pragma unroll
-        for (int m = 0; m < M; m++) a = a - val[m]*(m < nDep ? w[m] : T(0));
+        for (int m = 0; m < M; m++) a = a - val[m]*(W::lds || m < nDep ? w[m] : T(0));
         if (nDep > M)
         {
             const int32_t kLo = KIND == SWEEP_PRECOND_BWD ? nLo : BACKWARD ? nLo + M : M;
@@ -1129,8 +1190,9 @@ __device__ __forceinline__ void vf_rows(const RowsView& R, const SweepData<T>& d
             __hip_atomic_store(sync.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (st) st->scheduleError = 1;
         }
-        sw_st<true>(&wOut[r], a);
+        wOut.st(r, a);
     }
+    if constexpr (W::lds) __builtin_amdgcn_s_setprio(0);
 }
 
 template<class T, int KIND, bool BACKWARD>
@@ -1155,12 +1217,104 @@ void k_sweep_chunks_vf(RowsView R, SweepData<T> d, const T* wIn, T* wOut, ChunkV
         // slots: the dependencies (Gauss-Seidel forward: the others as well)
         const int32_t n = KIND == SWEEP_GS_FWD ? max(nLo, nEnt - nLo)
                         : BACKWARD ? nEnt - nLo : nLo;
-        if (!__any(n > 4)) vf_rows<T, KIND, BACKWARD, 4>(R, d, wIn, wOut, r, have, nLo, nEnt, sync, st);
-        else if (!__any(n > 8)) vf_rows<T, KIND, BACKWARD, 8>(R, d, wIn, wOut, r, have, nLo, nEnt, sync, st);
-        else if (!__any(n > 16)) vf_rows<T, KIND, BACKWARD, 16>(R, d, wIn, wOut, r, have, nLo, nEnt, sync, st);
-        else vf_rows<T, KIND, BACKWARD, 32>(R, d, wIn, wOut, r, have, nLo, nEnt, sync, st);
+        const VfGlobal<T> out{wOut};
+        if (!__any(n > 4)) vf_rows<T, KIND, BACKWARD, 4>(R, d, wIn, out, r, have, nLo, nEnt, sync, st);
+        else if (!__any(n > 8)) vf_rows<T, KIND, BACKWARD, 8>(R, d, wIn, out, r, have, nLo, nEnt, sync, st);
+        else if (!__any(n > 16)) vf_rows<T, KIND, BACKWARD, 16>(R, d, wIn, out, r, have, nLo, nEnt, sync, st);
+        else vf_rows<T, KIND, BACKWARD, 32>(R, d, wIn, out, r, have, nLo, nEnt, sync, st);
     }
 }
+
+// The same sweep by one workgroup with the values in LDS, for meshes that
+// fit there (GAMG coarse levels, small unstructured meshes): wavefront v
+// takes the chunks v, v + 8, ... in sweep order and polls its rows'
+// dependencies in LDS, so a level costs an LDS hand-off instead of one
+// through memory, and the matrix is streamed ahead by the wavefronts that
+// wait.  In place: values of the other side are read before the row, hence
+// before the rows that overwrite them.
+//
+// What bounds it: the critical path of a level -- the poll, the row's
+// values, its chain of products, the division -- in the code of one
+// wavefront, 0.33 us for DIC rows of one dependency, 0.6 for 8 to 15, 0.8
+// with a Gauss-Seidel row's other side (4, 8 and 12 wavefronts measured the
+// same until registers spilled; raised priority past the gate took 0.1 off).
+// Gauss-Seidel sweeps of the coarse levels of a 64 x 48 x 48 GAMG hierarchy
+// (us, before: one workgroup with a barrier per level, or through memory
+// from 16 rows a level on): 17756 rows in 315 levels 376 (489), 4431 in 197
+// 156 (300), 2213 in 152 121 (686), 553 in 80 65 (327), 33 in 15 14 (45).
+constexpr int VFL_WAVES = 8;
+template<class T, int KIND, bool BACKWARD>
+__global__ __launch_bounds__(VFL_WAVES*64)
+void k_sweep_chunks_lds(RowsView R, SweepData<T> d, int32_t nRows, ChunkView C, RowSync sync,
+                        DevState* st)
+{
+    __shared__ T vals[vf_lds_rows<T>() + 1];
+    __shared__ int done[VFL_WAVES];
+    if (st && st->done) return;
+    const int lane = (int)(threadIdx.x & 63);
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    for (int32_t i = (int32_t)threadIdx.x; i < nRows; i += VFL_WAVES*64)
+        vals[i] = SweepSentinel<T>::value();
+    if (threadIdx.x < VFL_WAVES) done[threadIdx.x] = -1;
+    if (threadIdx.x == 0) vals[vf_lds_rows<T>()] = T(0);
+    __syncthreads();
+    // a chunk's shape is read one turn ahead
+    int32_t r = 0, info = 0;
+    bool have = false;
+    auto shape = [&](int32_t q) {
+        have = false;
+        info = 0;
+        if (q >= C.nChunks) return;
+        const int32_t c = BACKWARD ? C.nChunks - 1 - q : q;
+        r = C.start[c] + lane;
+        have = r < C.start[c + 1];
+        info = have ? R.rowInfo[r] : 0;
+    };
+    shape(wave);
+    for (int32_t q = wave; q < C.nChunks; q += VFL_WAVES)
+    {
+        const int32_t r0 = r, nLo = info & 0xffff, nEnt = info >> 16;
+        const bool have0 = have;
+        shape(q + VFL_WAVES);
+        const VfLds<T> out{vals, d.w, &done[(q + VFL_WAVES - 2) % VFL_WAVES], q - 2};
+        const int32_t n = KIND == SWEEP_GS_FWD ? max(nLo, nEnt - nLo)
+                        : BACKWARD ? nEnt - nLo : nLo;
+        if (!__any(n > 4)) vf_rows<T, KIND, BACKWARD, 4>(R, d, d.w, out, r0, have0, nLo, nEnt, sync, st);
+        else if (!__any(n > 8)) vf_rows<T, KIND, BACKWARD, 8>(R, d, d.w, out, r0, have0, nLo, nEnt, sync, st);
+        else if (!__any(n > 12)) vf_rows<T, KIND, BACKWARD, 12>(R, d, d.w, out, r0, have0, nLo, nEnt, sync, st);
+        else vf_rows<T, KIND, BACKWARD, 16>(R, d, d.w, out, r0, have0, nLo, nEnt, sync, st);
+        if (lane == 0)
+            __hip_atomic_store(&done[wave], q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+}
+
+template<class T>
+bool launch_sweep_chunks_lds(int kind, const RowsView& R, const SweepData<T>& d, int32_t nRows,
+                             const ChunkView& C, const RowSync& sync, DevState* st,
+                             hipStream_t s)
+{
+    if (nRows > vf_lds_rows<T>()) return false;
+    const dim3 g(1), b(VFL_WAVES*64);
+    switch (kind)
+    {
+        case SWEEP_GS_FWD:
+            hipLaunchKernelGGL((k_sweep_chunks_lds<T, SWEEP_GS_FWD, false>), g, b, 0, s, R, d, nRows, C, sync, st);
+            return true;
+        case SWEEP_GS_BWD:
+            hipLaunchKernelGGL((k_sweep_chunks_lds<T, SWEEP_GS_BWD, true>), g, b, 0, s, R, d, nRows, C, sync, st);
+            return true;
+        case SWEEP_PRECOND_FWD:
+            hipLaunchKernelGGL((k_sweep_chunks_lds<T, SWEEP_PRECOND_FWD, false>), g, b, 0, s, R, d, nRows, C, sync, st);
+            return true;
+        case SWEEP_PRECOND_BWD:
+            hipLaunchKernelGGL((k_sweep_chunks_lds<T, SWEEP_PRECOND_BWD, true>), g, b, 0, s, R, d, nRows, C, sync, st);
+            return true;
+        default: return false;
+    }
+}
+
+template bool launch_sweep_chunks_lds<double>(int, const RowsView&, const SweepData<double>&, int32_t, const ChunkView&, const RowSync&, DevState*, hipStream_t);
+template bool launch_sweep_chunks_lds<float>(int, const RowsView&, const SweepData<float>&, int32_t, const ChunkView&, const RowSync&, DevState*, hipStream_t);
 
 template<class T, int KIND, bool BACKWARD>
 static void launch_rows_vf(const RowsView& R, const SweepData<T>& d, const T* wIn, T* wOut,

@@ -90,12 +90,12 @@ struct fh_matrix
     // pipelined sweep synchronisation
     fh::DBuf<unsigned long long> d_sync;  // [0] ticket, [1..nParts] progress
     unsigned long long epoch = 0;
-    // sync-free chunk sweeps (one-part meshes with wide levels)
+    // sync-free chunk sweeps (one-part meshes)
     fh::DBuf<unsigned int> d_rowFlags;     // per chunk
     fh::DBuf<unsigned long long> d_rowTicket;
     fh::DBuf<unsigned int> d_rowErr;
     unsigned long long rowTicketBase = 0, rowEpoch = 0, rowWaitTicks = 0;
-    bool rowSweep = false;
+    bool chunkSweeps = false;
     // output rows of the value-polling chunk passes that run in place
     fh::DBuf<double> d_chunkTmp;
     fh::DBuf<float> d_chunkTmp32;

@@ -349,10 +349,9 @@ void build_mesh(fh_mesh* m, int32_t nCells, int32_t nFaces,
                     fail(FH_ERR_INVALID, "internal: sweep order is not topological");
     }
 
-    // chunks of the sync-free sweep: used when the levels hold 16 rows or
-    // more on average (narrower dependency graphs, e.g. chains, are walked
-    // faster by the one-workgroup level sweep)
-    if (!m->tiled && nParts == 1 && (int64_t)nLevels*16 <= (int64_t)nCells)
+    // chunks of the sync-free sweeps
+    m->wideLevels = (int64_t)nLevels*16 <= (int64_t)nCells;
+    if (!m->tiled && nParts == 1)
     {
         std::vector<int32_t> start, chunkOf(nCells);
         for (size_t q = 0; q + 1 < S.segStart.size(); q++)
@@ -395,7 +394,6 @@ void build_mesh(fh_mesh* m, int32_t nCells, int32_t nFaces,
             fOff[c + 1] = (int32_t)fDeps.size();
             bOff[c + 1] = (int32_t)bDeps.size();
         }
-        m->chunkSweep = true;
         m->nChunks = nCh;
         m->d_chunkStart.upload(start, m->setupStream);
         m->d_fwdOff.upload(fOff, m->setupStream);

@@ -60,10 +60,10 @@ void matrix_init(fh_matrix* M, fh_mesh* mesh, hipStream_t shared)
     FH_HIP(hipMemsetAsync(M->d_finCount.p, 0, M->d_finCount.bytes(), M->stream));
     M->d_sync.alloc(1 + (size_t)mesh->sched.nParts);
     FH_HIP(hipMemsetAsync(M->d_sync.p, 0, M->d_sync.bytes(), M->stream));
-    // one-part meshes sweep row by row unless the level sweep is forced
+    // one-part meshes sweep by chunks unless the part sweep is forced
     const char* sw = std::getenv("FOAMHIP_SWEEP");
-    M->rowSweep = mesh->chunkSweep && !(sw && std::strcmp(sw, "parts") == 0);
-    if (M->rowSweep)
+    M->chunkSweeps = mesh->nChunks > 0 && !(sw && std::strcmp(sw, "parts") == 0);
+    if (M->chunkSweeps)
     {
         M->d_rowFlags.alloc(std::max(mesh->nChunks, 1));
         M->d_rowTicket.alloc(1);
@@ -259,32 +259,36 @@ static void sweep_any(fh_matrix* M, int kind, const SweepData<T>& d, DevState* s
         M->tileEpoch = ts.epoch;
         return;
     }
-    // one-part meshes (GAMG coarse levels, unstructured meshes): the
-    // multi-workgroup chunk sweep where the mesh has chunks (levels of 16
-    // rows or more on average), with each row's operands loaded before its
-    // chunk's wait, so a dependency level costs one flag hand-off and one
-    // round of value loads (GAMG levels of 7k-2M rows: 1.0-3.2 ms per
-    // Gauss-Seidel sweep against 1.5-43 ms for one workgroup);
-    // narrower dependency graphs (chains) are walked by one workgroup.
-    // FOAMHIP_SWEEP=chunks or parts forces the multi-workgroup sweeps.
-    static const bool multiWg = [] {
-        const char* e = std::getenv("FOAMHIP_SWEEP");
-        return e && (std::strcmp(e, "chunks") == 0 || std::strcmp(e, "parts") == 0);
-    }();
+    // one-part meshes (GAMG coarse levels, unstructured meshes): the chunk
+    // sweeps, polling the dependency values in LDS where the vector fits and
+    // one workgroup keeps up (an LDS level costs 0.5 to 0.8 us, one through
+    // memory 1.0 to 1.5, but a chunk takes one workgroup 0.3 us: 3.6 chunks
+    // a level, a 24^3 box with an obstacle, 79 against 78 us per
+    // Gauss-Seidel sweep; 1.4, 17756 coarse GAMG rows in 315 levels, 376
+    // against 489; 1, 2213 rows in 152 levels, 121 against 230), else in
+    // memory by persistent wavefronts.  The factor passes and the transposed
+    // one wait on chunk flags where the levels hold 16 rows or more on
+    // average, else one workgroup walks them.  FOAMHIP_SWEEP=chunks leaves
+    // out the LDS sweep, parts the chunk sweeps.
     const fh_mesh* mesh = M->mesh;
-    if (!multiWg && !mesh->chunkSweep && mesh->sched.nParts == 1 && mesh->nFaces > 0
-        && launch_sweep_level_wg<T>(kind, M->rows(), M->sched(), d, st, M->stream))
-        return;
-    if (M->rowSweep)
+    const bool polls = kind == SWEEP_GS_FWD || kind == SWEEP_GS_BWD || kind == SWEEP_PRECOND_FWD
+                    || kind == SWEEP_PRECOND_BWD;
+    if (M->chunkSweeps && (polls || mesh->wideLevels))
     {
-        RowSync rs = M->row_sync();
-        // the Gauss-Seidel and DIC/DILU passes poll the dependency values
-        // (three configuration-4 FP64 V-cycles: 0.146 s against 0.163 s with
-        // chunk flags); FOAMHIP_CHUNK_SYNC=flags waits on the chunk flags
+        static const bool inMemory = [] {
+            const char* e = std::getenv("FOAMHIP_SWEEP");
+            return e && std::strcmp(e, "chunks") == 0;
+        }();
+        // FOAMHIP_CHUNK_SYNC=flags waits on the chunk flags in all passes
         static const bool values = [] {
             const char* e = std::getenv("FOAMHIP_CHUNK_SYNC");
             return !(e && std::strcmp(e, "flags") == 0);
         }();
+        RowSync rs = M->row_sync();
+        if (values && !inMemory && (int64_t)mesh->nChunks <= 4*(int64_t)mesh->sched.nLevels
+            && launch_sweep_chunks_lds<T>(kind, M->rows(), d, mesh->nCells, M->chunks(), rs, st,
+                                          M->stream))
+            return;
         T* tmp = nullptr;
         if (values)
         {
@@ -1005,7 +1009,7 @@ void check_sweep_errors(fh_matrix* M)
             fail(FH_ERR_SCHEDULE, "a sweep dependency wait expired");
         }
     }
-    if (!M->rowSweep) return;
+    if (!M->d_rowErr.p) return;
     unsigned int e = 0;
     FH_HIP(hipMemcpyAsync(&e, M->d_rowErr.p, sizeof(e), hipMemcpyDeviceToHost, M->stream));
     FH_HIP(hipStreamSynchronize(M->stream));

@@ -1,6 +1,6 @@
-"""The value-polling chunk sweeps on layered graphs: rows with as many
-dependencies as their slots (4, 8, 16, 32), one more, and more than the
-largest, against the oracle's sequential loops."""
+"""The value-polling chunk sweeps, in LDS and in memory, on layered graphs:
+rows with as many dependencies as their slots (4, 8, 12, 16, 32), one more,
+and more than the largest, against the oracle's sequential loops."""
 import numpy as np
 import pytest
 
@@ -25,11 +25,37 @@ def layered(width, layers, deg, rng, spread):
 
 
 @pytest.mark.parametrize("deg,spread", [(1, False), (4, False), (5, True), (8, False), (9, True),
-                                        (16, False), (17, True), (32, False), (45, True)])
+                                        (12, False), (16, False), (17, True), (32, False),
+                                        (45, True)])
 @pytest.mark.parametrize("kind", ["spd", "asym"])
-def test_chunk_sweeps_bitwise(deg, spread, kind):
+@pytest.mark.parametrize("where", ["lds", "memory"])
+def test_chunk_sweeps_bitwise(deg, spread, kind, where):
     rng = np.random.default_rng(41 + deg)
-    n, lower, upper = layered(70 if deg < 32 else 130, 7, deg, rng, spread)
+    # more than 4 chunks a level go through memory
+    width = 300 if where == "memory" else 70 if deg < 32 else 130
+    n, lower, upper = layered(width, 7 if where == "lds" else 4, deg, rng, spread)
+    co = (spd_coeffs if kind == "spd" else asym_coeffs)(n, lower, upper, rng)
+    m = fh.lduMatrix(fh.lduAddressing(n, lower, upper), *co)
+    om = O.Matrix(O.Addr(n, lower, upper), *co)
+    psi, b = rng.standard_normal(n), rng.standard_normal(n)
+    for smoother in ("GaussSeidel", "symGaussSeidel"):
+        np.testing.assert_array_equal(m.smooth(smoother, psi, b, 2),
+                                      om.smooth(smoother, psi, b, 2))
+    precon = "DIC" if kind == "spd" else "DILU"
+    np.testing.assert_array_equal(m.precondition(precon, b), om.precondition(precon, b))
+
+
+@pytest.mark.parametrize("n", [1, 2, 300, 18432, 18433])
+@pytest.mark.parametrize("kind", ["spd", "asym"])
+def test_chain_and_lds_limit(n, kind):
+    """One row per level, up to the most rows the LDS sweep takes (FP64) and
+    one more, with a second diagonal so that a level reads two earlier ones."""
+    rng = np.random.default_rng(n)
+    i = np.arange(n, dtype=np.int32)
+    pairs = np.concatenate([np.stack([i[:-1], i[1:]], 1), np.stack([i[:-3], i[3:]], 1)]) \
+        if n > 3 else np.stack([i[:-1], i[1:]], 1)
+    pairs = pairs[np.lexsort((pairs[:, 1], pairs[:, 0]))]
+    lower, upper = pairs[:, 0].copy(), pairs[:, 1].copy()
     co = (spd_coeffs if kind == "spd" else asym_coeffs)(n, lower, upper, rng)
     m = fh.lduMatrix(fh.lduAddressing(n, lower, upper), *co)
     om = O.Matrix(O.Addr(n, lower, upper), *co)
