@@ -11,7 +11,7 @@ import pytest
 
 import foamhip as fh
 import oracle as O
-from meshes import asym_coeffs, box, random_graph, spd_coeffs
+from meshes import asym_coeffs, box, hub_graph, random_graph, spd_coeffs
 from test_gpu_solvers import ITER_TOL, SOLUTION_TOL, convdiff_case, laplacian_case, rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -654,3 +654,28 @@ def test_agglomeration_face_area_ties():
         np.testing.assert_array_equal(g["faceRestrict"], r["faceRestrict"])
         np.testing.assert_array_equal(g["lower"], r["lower"])
         np.testing.assert_array_equal(g["upper"], r["upper"])
+
+
+@pytest.mark.parametrize("name,gen", [
+    ("rand", lambda r: random_graph(3000, 6, r)),
+    ("sparse", lambda r: random_graph(900, 1.5, r, connect_chain=False)),
+    ("hubs", lambda r: hub_graph(2500, 3, 12, 40, r)),
+    ("box", lambda r: box(31, 26, 23)),
+])
+@pytest.mark.parametrize("smoother", ["GaussSeidel", "symGaussSeidel"])
+def test_colour_sweeps_in_lds(name, gen, smoother, monkeypatch):
+    """The FP32 colour sweeps of small levels in LDS and from memory are the
+    same operations in the same order: the same solution bits after the same
+    cycles (rows with more entries than the registers hold included)."""
+    rng = np.random.default_rng(61)
+    n, lower, upper = gen(rng)
+    diag, up = spd_coeffs(n, lower, upper, rng)
+    m = fh.lduMatrix(fh.lduAddressing(n, lower, upper), diag, up)
+    b = rng.uniform(-1, 1, n)
+    ctl = dict(GAMG, smoother=smoother, tolerance=1e-9, precision="mixed")
+    psi = [np.zeros(n), np.zeros(n)]
+    perf = fh.solver_New("p", m, ctl).solve(psi[0], b)
+    monkeypatch.setenv("FOAMHIP_COLOUR", "memory")
+    perf2 = fh.solver_New("p", m, ctl).solve(psi[1], b)
+    assert perf.converged and perf.nIterations == perf2.nIterations
+    assert np.array_equal(psi[0], psi[1])
