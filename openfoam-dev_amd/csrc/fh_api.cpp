@@ -569,8 +569,8 @@ int fh_h_device(fh_matrix* M, int32_t nCmpt, const double* d_psi, double* d_Hpsi
             FH_HIP(hipStreamSynchronize(M->stream));
             return;
         }
-        DBuf<double> x, y;
-        x.alloc((size_t)N*nCmpt); y.alloc((size_t)N*nCmpt);
+        DBuf<double>&x = M->callWork[0], &y = M->callWork[1];
+        x.reserve((size_t)N*nCmpt); y.reserve((size_t)N*nCmpt);
         launch_permute_cmpt_in(N, nCmpt, M->mesh->d_perm.p, d_psi, x.p, M->stream);
         launch_h(M->rows(), M->d_val.p, nCmpt, x.p, y.p, M->stream);
         launch_permute_cmpt_out(N, nCmpt, M->mesh->d_perm.p, y.p, d_Hpsi, M->stream);

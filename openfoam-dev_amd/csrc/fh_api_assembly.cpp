@@ -138,8 +138,8 @@ int fh_assemble_convection_diffusion(fh_matrix* M, const fh_boundary* b, const d
         M->d_diag.alloc(mesh->nCells);
         M->symmetric = false;
         M->diagonalOnly = false;
-        DBuf<double> work;
-        work.alloc(3*(size_t)F);
+        DBuf<double>& work = M->callWork[0];
+        work.reserve(3*(size_t)F);
         launch_convection_diffusion(M->rows(), mesh->d_perm.p, mesh->nFaces, b->view(), in,
                                     M->d_upperF.p, M->d_lowerF.p, work.p, M->d_diag.p, d_ic,
                                     d_bc, d_source, addBoundaryDiag, M->stream);
@@ -202,8 +202,9 @@ int fh_grad_gauss_linear(fh_mesh* mesh, const fh_boundary* b, const double* d_ph
         if (d_bGrad && b->nB && (!d_bMagSf || !d_bSnGrad))
             fail(FH_ERR_INVALID, "NULL boundary input for the patch gradient");
         GradInputs in{d_phi, d_weights, d_Sf, d_V, d_bSf, d_bMagSf, d_bPhi, d_bSnGrad};
-        DBuf<double> work;
-        work.alloc(3*(size_t)std::max(mesh->nFaces, 1));
+        std::lock_guard<std::mutex> lk(mesh->gradMutex);
+        DBuf<double>& work = mesh->gradWork;
+        work.reserve(3*(size_t)std::max(mesh->nFaces, 1));
         RowsView R;
         R.n = mesh->nCells;
         R.rowInfo = mesh->d_rowInfo.p;

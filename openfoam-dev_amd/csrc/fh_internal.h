@@ -6,6 +6,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -63,6 +64,11 @@ struct DBuf
         if (count == 0) return;
         FH_HIP(hipMalloc(&p, count*sizeof(T)));
         n = count;
+    }
+    // at least count values (workspaces kept between calls of several sizes)
+    void reserve(size_t count)
+    {
+        if (count > n) alloc(count);
     }
     void release()
     {
@@ -151,6 +157,13 @@ struct fh_mesh
     bool wideLevels = false;
     int32_t nChunks = 0;
     fh::DBuf<int32_t> d_chunkStart, d_fwdOff, d_fwdDeps, d_bwdOff, d_bwdDeps;
+
+    // face work of the gradients, kept with the mesh (an allocation and its
+    // release cost more than the kernels, and the release waits for the
+    // device); the lock is held over a call's launches and their end, as
+    // several threads may use the mesh
+    std::mutex gradMutex;
+    fh::DBuf<double> gradWork;
 
     // GAMG agglomeration cached with the mesh (built on the first GAMG
     // solve, as GAMGAgglomeration is cached on the mesh database)

@@ -96,6 +96,11 @@ struct fh_matrix
     fh::DBuf<unsigned int> d_rowErr;
     unsigned long long rowTicketBase = 0, rowEpoch = 0, rowWaitTicks = 0;
     bool chunkSweeps = false;
+    // work of single calls (coefficient updates, H, assembly), kept for the
+    // next one; every use is on the matrix's stream
+    fh::DBuf<double> callWork[2];
+    fh::DBuf<float> d_rounded;             // FP16-rounded coefficients (factor)
+    fh::DBuf<unsigned int> d_absRange;
     // output rows of the value-polling chunk passes that run in place
     fh::DBuf<double> d_chunkTmp;
     fh::DBuf<float> d_chunkTmp32;

@@ -55,7 +55,7 @@ struct Resident
 int64_t footprint_of(const fh_mesh* m)
 {
     const int64_t N = m->nCells, F = m->nFaces, nnz = m->nnzPad;
-    return 12*(N + nnz) + 16*F + 24*N + 40*N + 8*20*N + 4*12*N + (1 << 20)
+    return 12*(N + nnz) + 4*nnz + 8*N + 16*F + 24*N + 40*N + 8*20*N + 4*12*N + (1 << 20)
            + (m->tiled ? fh::march_bytes(m->boxNx, m->boxNy, m->boxNz) : 0);
 }
 

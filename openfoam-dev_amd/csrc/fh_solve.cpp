@@ -127,8 +127,8 @@ void matrix_set(fh_matrix* M, const double* diag, const double* upper, const dou
 
     M->diagonalOnly = (upper == nullptr);
     M->symmetric = (lower == nullptr);
-    DBuf<double> diagNat;
-    diagNat.alloc(N);
+    DBuf<double>& diagNat = M->callWork[0];
+    diagNat.reserve(N);
     FH_HIP(hipMemcpyAsync(diagNat.p, diag, sizeof(double)*N, kind, s));
     M->d_diag.alloc(N);
     launch_permute_in<double, double>(N, mesh->d_perm.p, diagNat.p, M->d_diag.p, s);
@@ -367,7 +367,7 @@ static bool tile_dic_half(fh_matrix* M)
     if (M->halfState == 0)
     {
         ensure_f32(M);
-        DBuf<unsigned int> range;
+        DBuf<unsigned int>& range = M->d_absRange;
         range.alloc(2);
         const unsigned int init[2] = {0u, 0xffffffffu};
         FH_HIP(hipMemcpyAsync(range.p, init, sizeof(init), hipMemcpyHostToDevice, M->stream));
@@ -418,7 +418,7 @@ const float* ensure_rD32(fh_matrix* M, int which)
         d.diag = M->d_diag32.p;
         d.w = b.p;
         d.upperF = M->d_upperF.p;
-        DBuf<float> rounded;
+        DBuf<float>& rounded = M->d_rounded;
         if (which == 3 && tile_dic_half(M))
         {
             const int64_t nnz = std::max<int64_t>(M->mesh->nnzPad, 1);
@@ -428,7 +428,6 @@ const float* ensure_rD32(fh_matrix* M, int which)
         }
         sweep_f(M, which == 4 ? SWEEP_RD_DILU : SWEEP_RD_DIC, d, nullptr, true);
         launch_reciprocal<float>(N, b.p, M->stream);
-        if (rounded.p) FH_HIP(hipStreamSynchronize(M->stream));
     }
     else
     {
