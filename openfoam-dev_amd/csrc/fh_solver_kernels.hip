@@ -727,11 +727,17 @@ int32_t launch_box_pcg_spmv(int32_t nx, int32_t ny, int32_t nz, const T* diag,
     }();
     if (!march)
     {
-        // slabs of 16 (FP32) / 8 (FP64) rows, about one block per CU
+        // slabs of 16 (FP32) / 8 (FP64) rows, about one block per CU (two in
+        // FP64); below 4 planes a run at most that many, as a block more per
+        // CU costs more than a plane more per run.  A plane of a run is a
+        // round trip and two barriers, so boxes smaller than the chip take
+        // runs of one (us per product, FP32 / FP64: 20^3 6.7 / 6.7 against
+        // 13.4 / 16.9 with runs of four, 64^3 7.0 / 10.7 against 12.6 / 12.4)
         constexpr int ROWS = sizeof(T) == 4 ? 16 : 8;
         const int64_t slabs = (int64_t)((nx + 255)/256)*((ny + ROWS - 1)/ROWS);
+        const int64_t most = sizeof(T) == 4 ? 256 : 512, planes = nz*slabs;
         const int32_t kc = (int32_t)std::max<int64_t>(
-            4, std::min<int64_t>(64, (int64_t)nz*slabs/(sizeof(T) == 4 ? 256 : 512)));
+            1, std::min<int64_t>(64, planes < 4*most ? (planes + most - 1)/most : planes/most));
         const int64_t runs = slabs*((nz + kc - 1)/kc);
         const int32_t nb = (int32_t)std::min<int64_t>(8*((runs + 7)/8), 2048);
         hipLaunchKernelGGL((k_box_spmv_slab<T, ROWS>), dim3(nb), dim3(64*ROWS), 0, s, nx, ny, nz,
