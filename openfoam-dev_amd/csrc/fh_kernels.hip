@@ -1208,7 +1208,7 @@ __device__ __forceinline__ void vf_rows(const RowsView& R, const SweepData<T>& d
     {
         if (KIND == SWEEP_PRECOND_FWD) a = b*a;
 #pragma unroll
-        for (int m = 0; m < M; m++) val[m] = b*val[m];
+        for (int m = 0; m < M; m++) val[m] = m < nDep ? b*val[m] : T(0);   // (b may be infinite)
     }
     // ---- the wait ----
     auto late = [&] {

@@ -65,3 +65,28 @@ def test_chain_and_lds_limit(n, kind):
                                       om.smooth(smoother, psi, b, 2))
     precon = "DIC" if kind == "spd" else "DILU"
     np.testing.assert_array_equal(m.precondition(precon, b), om.precondition(precon, b))
+
+
+@pytest.mark.parametrize("kind", ["spd", "asym"])
+@pytest.mark.parametrize("width", [40, 300])
+def test_infinite_factor_of_a_cell_without_faces(width, kind):
+    """A cell without faces and with a zero diagonal has an infinite factor:
+    its result is that factor times the residual, as it has no neighbour
+    values to take (in LDS, and in memory with the wider levels)."""
+    rng = np.random.default_rng(width)
+    n, lower, upper = layered(width, 5, 3, rng, True)
+    alone = np.array([0, n + 1], np.int32)          # two more cells, first and last
+    lower, upper = lower + 1, upper + 1
+    n += 2
+    co = list((spd_coeffs if kind == "spd" else asym_coeffs)(n, lower, upper, rng))
+    co[0][alone] = 0.0
+    m = fh.lduMatrix(fh.lduAddressing(n, lower, upper), *co)
+    om = O.Matrix(O.Addr(n, lower, upper), *co)
+    r = rng.standard_normal(n)
+    precon = "DIC" if kind == "spd" else "DILU"
+    ref = om.precondition(precon, r)
+    assert np.isinf(ref[alone]).all() and np.isfinite(np.delete(ref, alone)).all()
+    np.testing.assert_array_equal(m.precondition(precon, r), ref)
+    w = m.precondition_f32(precon, r)
+    np.testing.assert_array_equal(w[alone], ref[alone].astype(np.float32))
+    assert np.isfinite(np.delete(w, alone)).all()
