@@ -2,6 +2,7 @@
 // (fh_tile_march.hip).
 #pragma once
 
+#include "fh_march_shape.h"
 #include "fh_tile_sweep.h"
 
 namespace fh
@@ -22,26 +23,6 @@ struct MarchBufs
     DBuf<T> gsFwd, gsBwd, gsOld, gsPrime;
     bool gsFwdReady = false, gsBwdReady = false;
 };
-
-// Boxes the marching sweeps take: below 16 planes along k the padding of
-// the skewed coefficient order (21 steps per pencil) exceeds the cells
-// themselves; a vector with 64 planes beyond each end, and a pencil's halo
-// beyond the out-of-range mark, are within 32-bit byte offsets.
-constexpr int32_t kMarchMinNz = 16;
-inline bool march_fits(int32_t nx, int32_t ny, int32_t nz, int64_t valueBytes)
-{
-    return nz >= kMarchMinNz && nz <= (1 << 18)
-           && valueBytes*nx*ny*((int64_t)nz + 128) <= 0xE0000000ll;
-}
-
-// device bytes of all these buffers in FP64 (7 values per cell for DIC or
-// DILU, 11 and one unpadded for Gauss-Seidel, the halos)
-inline int64_t march_bytes(int32_t nx, int32_t ny, int32_t nz)
-{
-    if (!march_fits(nx, ny, nz, 8)) return 0;
-    const int64_t col = (int64_t)((nx + 15)/16)*((ny + 15)/16)*16;
-    return 8*(18*col*16*(nz + 36) + (int64_t)nx*ny*nz + 2*col*(nz + 16));
-}
 
 // packs dir (k, j, i coefficients of the pass, read at the neighbour with
 // dirShift) times rD for the forward or backward pass

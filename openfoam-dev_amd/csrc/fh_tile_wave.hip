@@ -1,6 +1,7 @@
 // One-wavefront tiled DIC / DILU sweeps for hex boxes: the global
 // preconditioner passes of boxes that the marching sweeps do not take
-// (fh_tile_march.hip: under 16 planes along k, or beyond 32-bit offsets).
+// (fh_tile_march.hip: under 16 planes along k, large boxes a few cells
+// thick, or beyond 32-bit offsets).
 //
 // The recurrences are those of fh_tile_sweep.hip (DICPreconditioner.C:
 // 87-123, DILUPreconditioner.C:88-135): cell (i,j,k) waits for its lower

@@ -88,3 +88,22 @@ def test_march_gauss_seidel_bitwise(size, kind, smoother):
     m.set(*co)
     om2 = O.Matrix(O.Addr(c.N, c.lower, c.upper), *co)
     np.testing.assert_array_equal(m.smooth(smoother, psi, b, 1), om2.smooth(smoother, psi, b, 1))
+
+
+@pytest.mark.parametrize("size", [(2, 2, 20000), (2, 2, 40000), (600, 2, 2000)])
+def test_thin_boxes(size):
+    """Boxes of which a pencil is mostly padding: up to a GiB of packed
+    coefficients they march, beyond that they stay on the tiles, whose
+    buffers are a few vectors."""
+    torch = pytest.importorskip("torch")
+    used = lambda: (lambda free, total: total - free)(*torch.cuda.mem_get_info())
+    c, rng, m, om = systems(size, "spd")
+    psi, r = rng.standard_normal(c.N), rng.standard_normal(c.N)
+    np.testing.assert_array_equal(m.precondition("diagonal", r), om.precondition("diagonal", r))
+    before = used()
+    np.testing.assert_array_equal(m.precondition("DIC", r), om.precondition("DIC", r))
+    np.testing.assert_array_equal(m.smooth("symGaussSeidel", psi, r, 1),
+                                  om.smooth("symGaussSeidel", psi, r, 1))
+    assert used() - before <= max(1 << 30, 4 * 18 * 8 * c.N)
+    if size == (2, 2, 40000):
+        assert used() - before <= 32 * 8 * c.N
