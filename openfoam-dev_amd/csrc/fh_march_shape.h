@@ -2,6 +2,8 @@
 // memory they hold for one.  Plain host code.
 #pragma once
 
+#include "foamhip.h"
+
 #include <cstdint>
 
 namespace fh
@@ -32,13 +34,70 @@ inline bool march_fits(int32_t nx, int32_t ny, int32_t nz, int64_t valueBytes)
            && (8*18*padded <= kMarchPaddedBytes || padded <= 4*((int64_t)nx*ny*nz));
 }
 
-// device bytes of all these buffers in FP64 (7 values per cell for DIC or
-// DILU, 11 and one unpadded for Gauss-Seidel, the halos)
-inline int64_t march_bytes(int32_t nx, int32_t ny, int32_t nz)
+// what a solve takes of them: the global DIC / DILU passes (FP64, FP32), the
+// Gauss-Seidel rows ascending and descending (FP64)
+enum : uint32_t { MARCH_DIC64 = 1, MARCH_DIC32 = 2, MARCH_GS_UP = 4, MARCH_GS_DOWN = 8 };
+
+inline uint32_t march_use_smoother(int32_t smoother, bool f32)
 {
-    if (!march_fits(nx, ny, nz, 8)) return 0;
-    const int64_t col = (int64_t)((nx + 15)/16)*((ny + 15)/16)*16;
-    return 8*(18*march_padded(nx, ny, nz) + (int64_t)nx*ny*nz + 2*col*(nz + 16));
+    const uint32_t dic = f32 ? MARCH_DIC32 : MARCH_DIC64;
+    // (the FP32 Gauss-Seidel sweeps run by colours)
+    const uint32_t up = f32 ? 0u : MARCH_GS_UP, down = f32 ? 0u : MARCH_GS_DOWN;
+    switch (smoother)
+    {
+        case FH_SMOOTH_GS: return up;
+        case FH_SMOOTH_SYMGS: return up | down;
+        case FH_SMOOTH_DIC:
+        case FH_SMOOTH_FDIC:
+        case FH_SMOOTH_DILU: return dic;
+        case FH_SMOOTH_DICGS:
+        case FH_SMOOTH_DILUGS: return dic | up;
+        default: return 0;
+    }
+}
+
+// the passes a solve with these controls runs on a box
+inline uint32_t march_use(const fh_controls& c)
+{
+    const bool krylov = c.solver == FH_SOLVER_PCG || c.solver == FH_SOLVER_PBICGSTAB
+                     || c.solver == FH_SOLVER_PBICG;
+    const bool f32 = c.precision == FH_PRECISION_MIXED && c.solver != FH_SOLVER_SMOOTH
+                  && c.solver != FH_SOLVER_PBICG;
+    if (!krylov)
+        return c.solver == FH_SOLVER_SMOOTH || c.solver == FH_SOLVER_GAMG
+               ? march_use_smoother(c.smoother, f32) : 0u;
+    int32_t p = c.preconditioner;
+    if (f32 && c.solver == FH_SOLVER_PCG)
+    {
+        // the inner preconditioner: tile-local in place of the global DIC
+        // unless one is asked for
+        if (c.innerPreconditioner >= 0) p = c.innerPreconditioner;
+        else if (p == FH_PRECON_DIC || p == FH_PRECON_FDIC) p = FH_PRECON_TILE_DIC;
+    }
+    if (p == FH_PRECON_DIC || p == FH_PRECON_FDIC || p == FH_PRECON_DILU)
+        return f32 ? MARCH_DIC32 : MARCH_DIC64;
+    if (p == FH_PRECON_GAMG)
+        return march_use_smoother((c.preconditionerControls ? c.preconditionerControls
+                                                            : &c)->smoother, f32);
+    return 0;
+}
+
+// device bytes of the buffers of these uses: 7 packed values per padded cell
+// for DIC or DILU, 7 and 4 for Gauss-Seidel and one vector, the halos
+inline int64_t march_bytes(int32_t nx, int32_t ny, int32_t nz, uint32_t use)
+{
+    const int64_t padded = march_padded(nx, ny, nz);
+    const int64_t halo = (int64_t)((nx + 15)/16)*((ny + 15)/16)*32*(nz + 16);
+    int64_t bytes = 0;
+    if ((use & ~MARCH_DIC32) && march_fits(nx, ny, nz, 8))
+    {
+        if (use & MARCH_DIC64) bytes += 8*7*padded;
+        if (use & MARCH_GS_UP) bytes += 8*7*padded;
+        if (use & MARCH_GS_DOWN) bytes += 8*4*padded + 8*(int64_t)nx*ny*nz;
+        bytes += 8*halo;
+    }
+    if ((use & MARCH_DIC32) && march_fits(nx, ny, nz, 4)) bytes += 4*(7*padded + halo);
+    return bytes;
 }
 
 } // namespace fh

@@ -10,8 +10,10 @@
 // Admission (in arrival order): a request runs when a slot is free and
 // either an idle resident matrix of its mesh exists or the estimated
 // footprint of a new one fits the memory budget -- after idle matrices of
-// other meshes are released, least recently used first.  A request larger
-// than the whole budget runs when nothing else is resident.
+// other meshes are released, least recently used first.  A resident matrix
+// whose earlier solves took fewer of the marching sweeps' buffers is priced
+// again.  A request larger than the whole budget runs when nothing else is
+// resident.
 #include "fh_matrix.h"
 
 #include <chrono>
@@ -39,6 +41,7 @@ struct Pending
     fh_controls precondControls{};     // owned copy of controls.preconditionerControls
     double submitTime = 0.0;
     int64_t footprint = 0;
+    uint32_t march = 0;                // the marching sweeps' buffers it uses
 };
 
 struct Resident
@@ -46,17 +49,23 @@ struct Resident
     fh_matrix* matrix = nullptr;
     fh_mesh* mesh = nullptr;
     int64_t bytes = 0;
+    uint32_t march = 0;                // buffers counted in bytes
 };
+
+int64_t march_of(const fh_mesh* m, uint32_t use)
+{
+    return m->tiled ? fh::march_bytes(m->boxNx, m->boxNy, m->boxNz, use) : 0;
+}
 
 // device bytes of one resident matrix with its solver work space: FP64 and
 // FP32 row values, face-ordered coefficients, packed FP32 tile
-// coefficients, factors and about twenty work vectors, and on a box the
-// buffers of the marching sweeps
-int64_t footprint_of(const fh_mesh* m)
+// coefficients, factors and about twenty work vectors (a 64^3 box solved by
+// mixed PCG holds 71 of the 107 MB), and on a box the buffers of the
+// marching sweeps it uses
+int64_t footprint_of(const fh_mesh* m, uint32_t march)
 {
     const int64_t N = m->nCells, F = m->nFaces, nnz = m->nnzPad;
-    return 12*(N + nnz) + 4*nnz + 8*N + 16*F + 24*N + 40*N + 8*20*N + 4*12*N + (1 << 20)
-           + (m->tiled ? fh::march_bytes(m->boxNx, m->boxNy, m->boxNz) : 0);
+    return 12*(N + nnz) + 16*F + 24*N + 40*N + 8*20*N + 4*12*N + (1 << 20) + march_of(m, march);
 }
 
 } // namespace
@@ -88,36 +97,45 @@ struct fh_server
     {
         if (queue.empty() || inFlight >= cfg.maxConcurrent) return false;
         Pending* p = queue.front().get();
+        // an idle matrix of this mesh, the one that lacks the least of the
+        // buffers the request uses
+        auto have = idle.end();
+        int64_t need = p->footprint;
         for (auto it = idle.begin(); it != idle.end(); ++it)
         {
-            if (it->mesh == p->mesh)
-            {
-                res = *it;
-                idle.erase(it);
-                job = std::move(queue.front());
-                queue.pop_front();
-                return true;
-            }
+            if (it->mesh != p->mesh) continue;
+            const int64_t more = march_of(p->mesh, it->march | p->march)
+                               - march_of(p->mesh, it->march);
+            if (have == idle.end() || more < need) { have = it; need = more; }
         }
-        // idle matrices (all of other meshes here) are released only when
-        // the request is admitted with it: a refused request frees nothing,
-        // so the bytes counted always match what is allocated
-        const int64_t need = p->footprint;
-        if (residentBytes + need > cfg.memoryBudget)
+        // the other idle matrices are released only when the request is
+        // admitted with it: a refused request frees nothing, so the bytes counted
+        // never fall below what the admitted requests are priced at
+        if (need > 0 && residentBytes + need > cfg.memoryBudget)
         {
             int64_t freeable = 0;
-            for (const Resident& r : idle) freeable += r.bytes;
+            for (auto it = idle.begin(); it != idle.end(); ++it)
+                if (it != have) freeable += it->bytes;
             if (residentBytes - freeable + need > cfg.memoryBudget && inFlight > 0)
                 return false;              // wait for a running solve to end
-            while (residentBytes + need > cfg.memoryBudget && !idle.empty())
+            for (auto it = idle.begin();
+                 it != idle.end() && residentBytes + need > cfg.memoryBudget;)
             {
-                release.push_back(idle.front());
-                residentBytes -= idle.front().bytes;
-                idle.pop_front();
+                if (it == have) { ++it; continue; }
+                release.push_back(*it);
+                residentBytes -= it->bytes;
+                it = idle.erase(it);
             }
         }
         residentBytes += need;
-        res = Resident{nullptr, p->mesh, need};
+        if (have != idle.end())
+        {
+            res = *have;
+            idle.erase(have);
+            res.bytes += need;
+            res.march |= p->march;
+        }
+        else res = Resident{nullptr, p->mesh, need, p->march};
         job = std::move(queue.front());
         queue.pop_front();
         return true;
@@ -248,7 +266,9 @@ int fh_server_submit(fh_server* s, const fh_request* r)
             job->precondControls.preconditionerControls = nullptr;
             job->controls.preconditionerControls = &job->precondControls;
         }
-        job->footprint = footprint_of(r->mesh);
+        // (without off-diagonal coefficients nothing is swept)
+        job->march = r->upper ? fh::march_use(job->controls) : 0u;
+        job->footprint = footprint_of(r->mesh, job->march);
         {
             std::lock_guard<std::mutex> lk(s->mu);
             if (s->solutions.count(r->id))

@@ -5,29 +5,44 @@ import subprocess
 
 import pytest
 
-CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
-                    "openfoam-dev_amd", "csrc")
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+MAIN = r"""
+#include "fh_march_shape.h"
+#include <cstdio>
+#include <cstdlib>
+// nx ny nz use: FP64 taken, FP32 taken, bytes; -1 solver preconditioner
+// smoother precision innerPreconditioner sub-smoother: the use
+int main(int n, char** s)
+{
+    int a[7];
+    for (int q = 1; q < n; q++) a[q - 1] = std::atoi(s[q]);
+    if (a[0] >= 0)
+        return std::printf("%d %d %lld\n", fh::march_fits(a[0], a[1], a[2], 8),
+                           fh::march_fits(a[0], a[1], a[2], 4),
+                           (long long)fh::march_bytes(a[0], a[1], a[2], a[3])) < 0;
+    fh_controls c{}, sub{};
+    c.solver = a[1]; c.preconditioner = a[2]; c.smoother = a[3]; c.precision = a[4];
+    c.innerPreconditioner = a[5];
+    sub.smoother = a[6];
+    if (a[6] >= 0) c.preconditionerControls = &sub;
+    return std::printf("%u\n", fh::march_use(c)) < 0;
+}
+"""
 
 
 @pytest.fixture(scope="module")
-def shape(tmp_path_factory):
-    """shape(nx, ny, nz) -> (taken in FP64, in FP32, device bytes)"""
+def call(tmp_path_factory):
     d = tmp_path_factory.mktemp("shape")
-    (d / "t.cpp").write_text(
-        '#include "fh_march_shape.h"\n#include <cstdio>\n#include <cstdlib>\n'
-        "int main(int, char** a) { int x = atoi(a[1]), y = atoi(a[2]), z = atoi(a[3]);\n"
-        'std::printf("%d %d %lld\\n", fh::march_fits(x, y, z, 8), fh::march_fits(x, y, z, 4),\n'
-        "(long long)fh::march_bytes(x, y, z)); }\n")
+    (d / "t.cpp").write_text(MAIN)
     exe = str(d / "t")
-    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(d / "t.cpp"), "-o",
-                    exe], check=True)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror",
+                    "-I", os.path.join(ROOT, "openfoam-dev_amd", "csrc"),
+                    "-I", os.path.join(ROOT, "include"), str(d / "t.cpp"), "-o", exe], check=True)
+    return lambda *a: [int(v) for v in subprocess.run(
+        [exe] + [str(v) for v in a], check=True, capture_output=True, text=True).stdout.split()]
 
-    def run(nx, ny, nz):
-        out = subprocess.run([exe, str(nx), str(ny), str(nz)], check=True, capture_output=True,
-                             text=True).stdout
-        f64, f32, b = out.split()
-        return bool(int(f64)), bool(int(f32)), int(b)
-    return run
+
+ALL = 1 | 4 | 8                # FP64: DIC, Gauss-Seidel ascending and descending
 
 
 @pytest.mark.parametrize("size,taken", [
@@ -37,9 +52,52 @@ def shape(tmp_path_factory):
     # mostly padding: both sides of 1 GiB, and of 4 times the cells beyond it
     ((2, 2, 29000), True), ((2, 2, 29200), False), ((4000, 2, 2000), False),
     ((2, 2, 200000), False), ((5, 1000, 1000), True), ((3, 1000, 1000), False)])
-def test_boxes_taken(shape, size, taken):
-    f64, f32, b = shape(*size)
+def test_boxes_taken(call, size, taken):
+    f64, f32, b = call(*size, ALL)
     assert f64 == taken and (b > 0) == taken
     assert f32 or not f64
     # what the padding may cost
     assert b <= max((1 << 30) + (1 << 27), 600 * size[0] * size[1] * size[2])
+
+
+PRECON = {"none": 0, "diagonal": 1, "DIC": 2, "FDIC": 3, "DILU": 4, "GAMG": 5, "tileDIC": 6}
+SMOOTH = {"GaussSeidel": 0, "symGaussSeidel": 1, "DIC": 2, "DILU": 3, "DICGaussSeidel": 4}
+PCG, BICGSTAB, BICG, SWEEPS, MULTIGRID, DIAGONAL = range(6)
+DIC64, DIC32, UP, DOWN = 1, 2, 4, 8
+
+
+@pytest.mark.parametrize("solver,precon,smoother,mixed,inner,sub,use", [
+    (PCG, "DIC", "GaussSeidel", 0, None, None, DIC64), (PCG, "FDIC", "DIC", 0, None, None, DIC64),
+    (PCG, "diagonal", "DIC", 0, None, None, 0), (PCG, "none", "DIC", 1, None, None, 0),
+    # mixed PCG: tile-local unless another inner preconditioner is asked for
+    (PCG, "DIC", "DIC", 1, None, None, 0), (PCG, "DIC", "DIC", 1, "DIC", None, DIC32),
+    (PCG, "tileDIC", "DIC", 0, None, None, 0), (PCG, "DIC", "DIC", 1, "tileDIC", None, 0),
+    (BICGSTAB, "DILU", "DIC", 0, None, None, DIC64),
+    (BICGSTAB, "DILU", "DIC", 1, None, None, DIC32), (BICG, "DILU", "DIC", 1, None, None, DIC64),
+    (SWEEPS, "none", "GaussSeidel", 0, None, None, UP),
+    (SWEEPS, "none", "symGaussSeidel", 1, None, None, UP | DOWN),
+    (SWEEPS, "none", "DILU", 0, None, None, DIC64),
+    (SWEEPS, "none", "DICGaussSeidel", 0, None, None, DIC64 | UP),
+    (MULTIGRID, "none", "symGaussSeidel", 0, None, None, UP | DOWN),
+    (MULTIGRID, "none", "symGaussSeidel", 1, None, None, 0),
+    (MULTIGRID, "none", "DICGaussSeidel", 1, None, None, DIC32),
+    (PCG, "GAMG", "DIC", 0, None, "GaussSeidel", UP),
+    (PCG, "GAMG", "GaussSeidel", 1, None, "DIC", DIC32),
+    (DIAGONAL, "DIC", "DIC", 0, None, None, 0)])
+def test_what_a_solve_uses(call, solver, precon, smoother, mixed, inner, sub, use):
+    assert call(-1, solver, PRECON[precon], SMOOTH[smoother], mixed,
+                PRECON[inner] if inner else -1, SMOOTH[sub] if sub else -1) == [use]
+
+
+@pytest.mark.parametrize("size", [(64, 64, 64), (17, 33, 19)])
+def test_bytes_by_use(call, size):
+    nx, ny, nz = size
+    cols = -(-nx // 16) * -(-ny // 16) * 256
+    packed, halo = cols * (nz + 36), cols // 8 * (nz + 16)
+    at = lambda use: call(nx, ny, nz, use)[2]
+    assert at(0) == 0
+    assert at(DIC64) == 8 * (7 * packed + halo) and at(DIC32) == 4 * (7 * packed + halo)
+    assert at(UP) == 8 * (7 * packed + halo)
+    assert at(UP | DOWN) == 8 * (11 * packed + nx * ny * nz + halo)
+    assert at(ALL) == 8 * (18 * packed + nx * ny * nz + halo)
+    assert at(ALL | DIC32) == at(ALL) + at(DIC32)
