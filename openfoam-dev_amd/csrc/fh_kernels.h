@@ -145,8 +145,13 @@ struct RowSync
     unsigned long long epoch;          // launches made with this context
     unsigned long long waitTicks;      // wall-clock bound of one wait
     unsigned int* err;                 // set when a wait expired
+    int32_t perLevel = 0;              // chunks per level, on average
 };
 
+// chunks per level times the rows' slots from which on the value-polling
+// sweep waits for a chunk's last dependency before it loads them all
+// (k_sweep_chunks_vf)
+constexpr int32_t kVfLastDep = 1000;
 // LDS of the one-workgroup chunk sweep, and the rows that fit there
 constexpr int32_t kVfLdsBytes = 144*1024;
 template<class T> constexpr int32_t vf_lds_rows() { return kVfLdsBytes/(int32_t)sizeof(T); }

@@ -1105,6 +1105,16 @@ void k_sweep_chunks(RowsView R, SweepData<T> d, ChunkView C, RowSync sync,
 // with an obstacle): 204 us forward, 217 backward, 0.95 us a level, which is
 // one hand-off through memory; with one lane polling the latest dependency
 // before the rows loaded theirs, and 32 slots for every row, 564 and 606.
+//
+// Polling every dependency multiplies the loads of a level by the rounds of
+// polling, which pays while they are few.  With 32 slots, or where the
+// chunks per level times the slots reach kVfLastDep, the gate is the chunk's
+// last dependency itself and only what is not there after it is loaded
+// again.  Both ways, us for a forward DIC pass: 27 chunks a level, 4 slots,
+// 213 polling / 266 behind the last (the box above); 202 chunks (a 200^3 box
+// with an obstacle) 1604 / 1664; 313 chunks, random neighbours, 120 / 96; 18
+// chunks, 16 slots, a GAMG level, 949 / 1276; 63 chunks, random, 138 / 98;
+// 313 chunks, 32 slots, 391 / 151 (Gauss-Seidel forward 3170 / 394).
 // --------------------------------------------------------------------------
 // the fill and the copy back do nothing once the solve is done, like the
 // pass itself (which then computes no row)
@@ -1175,7 +1185,9 @@ __device__ __forceinline__ void vf_rows(const RowsView& R, const SweepData<T>& d
         for (int off = 32; off > 0; off >>= 1) key = max(key, __shfl_xor(key, off, 64));
         kr = __builtin_amdgcn_readfirstlane(BACKWARD ? -key : key);
     }
-    if (!W::lds && anyDep)
+    const bool last = !W::lds && (M >= 32 || sync.perLevel*M >= kVfLastDep);
+    if (last && anyDep) gate = BACKWARD ? -kr : kr;
+    if (!W::lds && !last && anyDep)
     {
         const int32_t info = R.rowInfo[kr];
         const int32_t kLo = info & 0xffff, kEnt = info >> 16;
@@ -1268,7 +1280,26 @@ __device__ __forceinline__ void vf_rows(const RowsView& R, const SweepData<T>& d
                 }
             } while (p);
         }
-        else
+        else if (last)
+        {
+            // what has not been written yet is loaded again, alone
+#pragma unroll
+            for (int m = 0; m < M; m++) w[m] = m < nDep ? wOut.ld(col[m]) : T(0);
+            for (;;)
+            {
+                asm volatile("" ::: "memory");
+                bool p = false;
+#pragma unroll
+                for (int m = 0; m < M; m++) p |= S::is(w[m]);
+                if (!__any(p)) break;
+                if (__any(expired || late())) { expired = true; break; }
+                __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+                for (int m = 0; m < M; m++)
+                    if (S::is(w[m])) w[m] = wOut.ld(col[m]);
+            }
+        }
+        else if constexpr (M < 32)
         {
             T u[M];
             sample(w);

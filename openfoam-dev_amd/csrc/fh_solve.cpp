@@ -285,6 +285,7 @@ static void sweep_any(fh_matrix* M, int kind, const SweepData<T>& d, DevState* s
             return !(e && std::strcmp(e, "flags") == 0);
         }();
         RowSync rs = M->row_sync();
+        rs.perLevel = mesh->nChunks/std::max(mesh->sched.nLevels, 1);
         if (values && !inMemory && (int64_t)mesh->nChunks <= 4*(int64_t)mesh->sched.nLevels
             && launch_sweep_chunks_lds<T>(kind, M->rows(), d, mesh->nCells, M->chunks(), rs, st,
                                           M->stream))

@@ -90,3 +90,26 @@ def test_infinite_factor_of_a_cell_without_faces(width, kind):
     w = m.precondition_f32(precon, r)
     np.testing.assert_array_equal(w[alone], ref[alone].astype(np.float32))
     assert np.isfinite(np.delete(w, alone)).all()
+
+
+@pytest.mark.parametrize("width,deg", [(15900, 3), (16100, 3), (8100, 8), (4100, 12), (2100, 30)])
+@pytest.mark.parametrize("kind", ["spd", "asym"])
+def test_wide_levels_bitwise(width, deg, kind):
+    """Levels of many chunks, where the rows wait for a chunk's last
+    dependency before they load them all (4, 8, 16 and 32 slots; just under
+    the first limit, too)."""
+    rng = np.random.default_rng(width)
+    c = np.arange(width)
+    hop = rng.choice(np.arange(1, width), deg, replace=False)
+    pairs = np.concatenate([np.stack([l * width + (c + h) % width, (l + 1) * width + c], 1)
+                            for l in range(3) for h in hop]).astype(np.int32)
+    pairs = pairs[np.lexsort((pairs[:, 1], pairs[:, 0]))]
+    n, lower, upper = 4 * width, pairs[:, 0].copy(), pairs[:, 1].copy()
+    co = (spd_coeffs if kind == "spd" else asym_coeffs)(n, lower, upper, rng)
+    m = fh.lduMatrix(fh.lduAddressing(n, lower, upper), *co)
+    om = O.Matrix(O.Addr(n, lower, upper), *co)
+    psi, b = rng.standard_normal(n), rng.standard_normal(n)
+    np.testing.assert_array_equal(m.smooth("symGaussSeidel", psi, b, 2),
+                                  om.smooth("symGaussSeidel", psi, b, 2))
+    precon = "DIC" if kind == "spd" else "DILU"
+    np.testing.assert_array_equal(m.precondition(precon, b), om.precondition(precon, b))
