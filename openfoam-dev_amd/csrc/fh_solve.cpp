@@ -261,15 +261,23 @@ static void sweep_any(fh_matrix* M, int kind, const SweepData<T>& d, DevState* s
     }
     // one-part meshes (GAMG coarse levels, unstructured meshes): the chunk
     // sweeps, polling the dependency values in LDS where the vector fits and
-    // one workgroup keeps up (an LDS level costs 0.5 to 0.8 us, one through
-    // memory 1.0 to 1.5, but a chunk takes one workgroup 0.3 us: 3.6 chunks
-    // a level, a 24^3 box with an obstacle, 79 against 78 us per
-    // Gauss-Seidel sweep; 1.4, 17756 coarse GAMG rows in 315 levels, 376
-    // against 489; 1, 2213 rows in 152 levels, 121 against 230), else in
-    // memory by persistent wavefronts.  The factor passes and the transposed
-    // one wait on chunk flags where the levels hold 16 rows or more on
-    // average, else one workgroup walks them.  FOAMHIP_SWEEP=chunks leaves
-    // out the LDS sweep, parts the chunk sweeps.
+    // one workgroup keeps up, else in memory by persistent wavefronts.  An
+    // LDS level costs 0.4 to 0.8 us, one through memory 1.0 to 1.5, but one
+    // workgroup takes 0.3 us for a chunk of few entries and more for many:
+    // it is taken up to 30 entries a row (those the pass takes: Gauss-Seidel
+    // all, DIC / DILU one side) times the chunks per level, and up to 3
+    // chunks a level (DIC / DILU 4, and with few chunks whatever the rows
+    // hold).  In LDS / in memory, us per forward
+    // Gauss-Seidel sweep and DIC pass: GAMG levels of 1.4 chunks, 13 entries
+    // 378 / 458 and 186 / 345; 1 chunk, 15 entries 204 / 367 and 152 / 275;
+    // a 24^3 box with an obstacle, 3.6 chunks, 6 entries 82 / 76 and 55 / 62;
+    // graphs of 1 chunk, 25 entries 271 / 339 and 65 / 120, 40 entries
+    // 487 / 343 and 172 / 246, 119 entries 5942 / 5090 and 1288 / 2337; 2 chunks, 53 entries 1092 / 604 and 214 / 263; 4
+    // chunks, 6 entries 131 / 103 and 60 / 67, 56 entries 1629 / 471 and
+    // 308 / 169.  The factor passes and the transposed one wait on chunk
+    // flags where the levels hold 16 rows or more on average, else one
+    // workgroup walks them.  FOAMHIP_SWEEP=chunks leaves out the LDS sweep,
+    // parts the chunk sweeps.
     const fh_mesh* mesh = M->mesh;
     const bool polls = kind == SWEEP_GS_FWD || kind == SWEEP_GS_BWD || kind == SWEEP_PRECOND_FWD
                     || kind == SWEEP_PRECOND_BWD;
@@ -286,7 +294,13 @@ static void sweep_any(fh_matrix* M, int kind, const SweepData<T>& d, DevState* s
         }();
         RowSync rs = M->row_sync();
         rs.perLevel = mesh->nChunks/std::max(mesh->sched.nLevels, 1);
-        if (values && !inMemory && (int64_t)mesh->nChunks <= 4*(int64_t)mesh->sched.nLevels
+        const bool gs = kind == SWEEP_GS_FWD || kind == SWEEP_GS_BWD;
+        const double levels = mesh->sched.nLevels, chunks = mesh->nChunks;
+        const double entries = (gs ? 2.0 : 1.0)*mesh->nFaces/std::max(mesh->nCells, 1);
+        const bool oneKeepsUp = gs ? chunks <= 3*levels && chunks*entries <= 30*levels
+                                   : chunks <= 4*levels && (chunks*entries <= 30*levels
+                                                            || chunks <= 1.5*levels);
+        if (values && !inMemory && oneKeepsUp
             && launch_sweep_chunks_lds<T>(kind, M->rows(), d, mesh->nCells, M->chunks(), rs, st,
                                           M->stream))
             return;

@@ -113,3 +113,29 @@ def test_wide_levels_bitwise(width, deg, kind):
                                   om.smooth("symGaussSeidel", psi, b, 2))
     precon = "DIC" if kind == "spd" else "DILU"
     np.testing.assert_array_equal(m.precondition(precon, b), om.precondition(precon, b))
+
+
+@pytest.mark.parametrize("deg", [16, 17, 40])
+@pytest.mark.parametrize("kind", ["spd", "asym"])
+def test_few_rows_of_many_entries_in_lds(deg, kind):
+    """The LDS sweep's rows past its 16 slots: few enough of them that the
+    mesh stays in LDS (a chain of 64-cell levels with hubs of deg lower and
+    deg upper neighbours)."""
+    rng = np.random.default_rng(deg)
+    width, layers = 64, 24
+    pairs = {((l - 1) * width + c, l * width + c) for l in range(1, layers) for c in range(width)}
+    for l in range(1, layers - 1, 3):
+        hub = l * width + int(rng.integers(width))
+        pairs |= {((l - 1) * width + int(p), hub) for p in rng.choice(width, deg, replace=False)}
+        pairs |= {(hub, (l + 1) * width + int(p)) for p in rng.choice(width, deg, replace=False)}
+    pairs = np.array(sorted(pairs), dtype=np.int32)
+    n, lower, upper = width * layers, pairs[:, 0].copy(), pairs[:, 1].copy()
+    co = (spd_coeffs if kind == "spd" else asym_coeffs)(n, lower, upper, rng)
+    m = fh.lduMatrix(fh.lduAddressing(n, lower, upper), *co)
+    om = O.Matrix(O.Addr(n, lower, upper), *co)
+    psi, b = rng.standard_normal(n), rng.standard_normal(n)
+    for smoother in ("GaussSeidel", "symGaussSeidel"):
+        np.testing.assert_array_equal(m.smooth(smoother, psi, b, 2),
+                                      om.smooth(smoother, psi, b, 2))
+    precon = "DIC" if kind == "spd" else "DILU"
+    np.testing.assert_array_equal(m.precondition(precon, b), om.precondition(precon, b))

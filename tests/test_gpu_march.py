@@ -12,7 +12,7 @@ from meshes import asym_coeffs, spd_coeffs
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [(1, 1, 16), (5, 3, 70), (16, 16, 16), (17, 33, 19), (16, 64, 63), (40, 18, 133),
+SIZES = [(2, 2, 16), (2, 3, 70), (5, 3, 70), (16, 16, 16), (17, 33, 19), (16, 64, 63), (40, 18, 133),
          (33, 47, 64), (270, 270, 17)]
 
 
@@ -21,6 +21,7 @@ def systems(size, kind, seed=5):
     rng = np.random.default_rng(seed)
     a = O.Addr(c.N, c.lower, c.upper)
     mesh = fh.lduAddressing(c.N, c.lower, c.upper)
+    assert mesh.info()["tiled"]
     if kind == "spd":
         co = spd_coeffs(c.N, c.lower, c.upper, rng)
     else:
