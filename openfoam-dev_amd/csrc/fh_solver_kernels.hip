@@ -700,6 +700,29 @@ static int32_t box_x4_blocks(int32_t nx, int32_t ny, int32_t nz)
     return (int32_t)std::min<int64_t>(8*((nb4 + 7)/8), 2048);
 }
 
+// Planes of a run of the slab product.  A CU takes one run at a time (the
+// second block of a CU costs what a second round does), and a run of kc
+// planes about kc + 2 steps, each a round trip and two barriers: the kc of
+// fewest steps over the rounds of 256 runs, the longer one of two (it reads
+// fewer planes of p twice).  us per product, FP32 / FP64, with this rule and
+// with the other choices: 20^3 6.8 / 6.8 (runs of one; of four 13.8 / 17.1),
+// 64^3 7.1 / 8.4 (1 and 2 planes; 4: 12.7 / 12.4, FP64 1: 10.6), 200 x 152
+// x 40 11.4 / 18.5 (2 and 4 planes; FP64 2: 21.4), 256 x 2000 x 3 16.3 /
+// 20.7 (2 and 3; FP64 2: 27.7), 512 x 800 x 3 13.2 / 18.4 (FP64 2: 24.5),
+// 200^3 47 / 110 (11 and 20; 10: 72, 9: 134), 300^3 270 / 522 (50 and 30;
+// 44: 425 and 679).
+static int32_t box_slab_run(int64_t slabs, int32_t nz)
+{
+    int32_t best = 1;
+    int64_t fewest = INT64_MAX;
+    for (int32_t kc = 1; kc <= std::min(nz, 64); kc++)
+    {
+        const int64_t rounds = (slabs*((nz + kc - 1)/kc) + 255)/256;
+        if (rounds*(kc + 2) <= fewest) { fewest = rounds*(kc + 2); best = kc; }
+    }
+    return best;
+}
+
 template<class T>
 int32_t launch_box_pcg_spmv(int32_t nx, int32_t ny, int32_t nz, const T* diag,
                             const T* const dir[6], bool symmetric, const T* w,
@@ -727,17 +750,10 @@ int32_t launch_box_pcg_spmv(int32_t nx, int32_t ny, int32_t nz, const T* diag,
     }();
     if (!march)
     {
-        // slabs of 16 (FP32) / 8 (FP64) rows, about one block per CU (two in
-        // FP64); below 4 planes a run at most that many, as a block more per
-        // CU costs more than a plane more per run.  A plane of a run is a
-        // round trip and two barriers, so boxes smaller than the chip take
-        // runs of one (us per product, FP32 / FP64: 20^3 6.7 / 6.7 against
-        // 13.4 / 16.9 with runs of four, 64^3 7.0 / 10.7 against 12.6 / 12.4)
+        // slabs of 16 (FP32) / 8 (FP64) rows, in runs of kc planes
         constexpr int ROWS = sizeof(T) == 4 ? 16 : 8;
         const int64_t slabs = (int64_t)((nx + 255)/256)*((ny + ROWS - 1)/ROWS);
-        const int64_t most = sizeof(T) == 4 ? 256 : 512, planes = nz*slabs;
-        const int32_t kc = (int32_t)std::max<int64_t>(
-            1, std::min<int64_t>(64, planes < 4*most ? (planes + most - 1)/most : planes/most));
+        const int32_t kc = box_slab_run(slabs, nz);
         const int64_t runs = slabs*((nz + kc - 1)/kc);
         const int32_t nb = (int32_t)std::min<int64_t>(8*((runs + 7)/8), 2048);
         hipLaunchKernelGGL((k_box_spmv_slab<T, ROWS>), dim3(nb), dim3(64*ROWS), 0, s, nx, ny, nz,

@@ -224,3 +224,24 @@ def test_mixed_precision_vs_fp64_oracle(solver, precon):
     assert perf2.converged
     opsi2, _ = om.solve(tight, np.zeros(c.N), b)
     assert rel_l2(psi2, opsi2) <= MIXED_TOL
+
+
+@pytest.mark.parametrize("size", [(4, 2, 2), (260, 9, 5), (64, 2000, 3), (8, 9, 260), (8, 20, 700),
+                                  (4, 130, 140), (12, 4100, 2)])
+def test_pcg_product_runs(size):
+    """The box product at its lengths of a run: one plane, all planes, some
+    with a shorter last run, and more slabs than compute units."""
+    from meshes import spd_coeffs
+    c = BoxCase(*size)
+    rng = np.random.default_rng(sum(size))
+    diag, upper = spd_coeffs(c.N, c.lower, c.upper, rng)
+    a, b = O.Addr(c.N, c.lower, c.upper), rng.uniform(-1, 1, c.N)
+    om = O.Matrix(a, diag, upper)
+    m = fh.lduMatrix(fh.lduAddressing(c.N, c.lower, c.upper), diag, upper)
+    ctl = {"solver": "PCG", "preconditioner": "diagonal", "tolerance": 1e-11, "relTol": 0}
+    opsi, operf = om.solve(ctl, np.zeros(c.N), b)
+    psi = np.zeros(c.N)
+    compare(fh.solver_New("p", m, ctl).solve(psi, b), opsi, psi, operf)
+    psi = np.zeros(c.N)
+    perf = fh.solver_New("p", m, dict(ctl, precision="mixed")).solve(psi, b)
+    assert perf.converged and rel_l2(psi, opsi) <= MIXED_TOL
