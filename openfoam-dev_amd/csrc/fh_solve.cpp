@@ -571,14 +571,12 @@ template<> void sweep_t<float>(fh_matrix* M, int kind, const SweepData<float>& d
     sweep_f(M, kind, d, st, local);
 }
 
-// FOAMHIP_BOX_SWEEP: 0 default, 1 wide, 2 wave
+// FOAMHIP_BOX_SWEEP: 0 default, 1 wide, 2 wave (read at every pass, so a
+// process can switch between them)
 static int box_sweep_forced()
 {
-    static const int forced = [] {
-        const char* e = std::getenv("FOAMHIP_BOX_SWEEP");
-        return !e ? 0 : std::strcmp(e, "wide") == 0 ? 1 : std::strcmp(e, "wave") == 0 ? 2 : 0;
-    }();
-    return forced;
+    const char* e = std::getenv("FOAMHIP_BOX_SWEEP");
+    return !e ? 0 : std::strcmp(e, "wide") == 0 ? 1 : std::strcmp(e, "wave") == 0 ? 2 : 0;
 }
 
 template<class T> static MarchBufs<T>& march_bufs(fh_matrix* M);

@@ -12,7 +12,7 @@ from meshes import asym_coeffs, spd_coeffs
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [(2, 2, 16), (2, 3, 70), (5, 3, 70), (16, 16, 16), (17, 33, 19), (16, 64, 63), (40, 18, 133),
+SIZES = [(1, 1, 16), (5, 3, 70), (16, 16, 16), (17, 33, 19), (16, 64, 63), (40, 18, 133),
          (33, 47, 64), (270, 270, 17)]
 
 
@@ -21,7 +21,6 @@ def systems(size, kind, seed=5):
     rng = np.random.default_rng(seed)
     a = O.Addr(c.N, c.lower, c.upper)
     mesh = fh.lduAddressing(c.N, c.lower, c.upper)
-    assert mesh.info()["tiled"]
     if kind == "spd":
         co = spd_coeffs(c.N, c.lower, c.upper, rng)
     else:
@@ -89,6 +88,26 @@ def test_march_gauss_seidel_bitwise(size, kind, smoother):
     m.set(*co)
     om2 = O.Matrix(O.Addr(c.N, c.lower, c.upper), *co)
     np.testing.assert_array_equal(m.smooth(smoother, psi, b, 1), om2.smooth(smoother, psi, b, 1))
+
+
+@pytest.mark.parametrize("box_sweep", ["wave", "wide"])
+@pytest.mark.parametrize("size", [(2, 3, 70), (17, 33, 19), (40, 18, 133), (33, 47, 64)])
+@pytest.mark.parametrize("kind", ["spd", "asym"])
+def test_tiles_of_many_planes_bitwise(size, kind, box_sweep, monkeypatch):
+    """The tile kernels that boxes beyond the marching sweeps' limits take,
+    with tiles waiting on tiles along k as well, and the pencils between
+    them on the same matrix."""
+    c, rng, m, om = systems(size, kind)
+    precon = "DIC" if kind == "spd" else "DILU"
+    psi, r = rng.standard_normal(c.N), rng.standard_normal(c.N)
+    ref = om.precondition(precon, r), om.smooth("symGaussSeidel", psi, r, 2)
+    march32 = m.precondition_f32(precon, r)
+    for forced in (box_sweep, "", box_sweep):
+        monkeypatch.setenv("FOAMHIP_BOX_SWEEP", forced)
+        np.testing.assert_array_equal(m.precondition(precon, r), ref[0])
+        np.testing.assert_array_equal(m.smooth("symGaussSeidel", psi, r, 2), ref[1])
+    # the same operations in FP32
+    np.testing.assert_array_equal(m.precondition_f32(precon, r), march32)
 
 
 @pytest.mark.parametrize("size", [(2, 2, 20000), (2, 2, 40000), (600, 2, 2000)])
