@@ -12,7 +12,7 @@ from meshes import asym_coeffs, spd_coeffs
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [(1, 1, 16), (5, 3, 70), (16, 16, 16), (17, 33, 19), (16, 64, 63), (40, 18, 133),
+SIZES = [(2, 2, 17), (2, 3, 70), (5, 3, 70), (16, 16, 16), (17, 33, 19), (16, 64, 63), (40, 18, 133),
          (33, 47, 64), (270, 270, 17)]
 
 
@@ -21,6 +21,7 @@ def systems(size, kind, seed=5):
     rng = np.random.default_rng(seed)
     a = O.Addr(c.N, c.lower, c.upper)
     mesh = fh.lduAddressing(c.N, c.lower, c.upper)
+    assert mesh.info()["tiled"]
     if kind == "spd":
         co = spd_coeffs(c.N, c.lower, c.upper, rng)
     else:
@@ -38,15 +39,16 @@ def test_march_precondition_bitwise(size, kind, precon):
 
 
 @pytest.mark.parametrize("size", SIZES[:6])
-def test_march_f32(size):
+@pytest.mark.parametrize("kind,precon", [("spd", "DIC"), ("asym", "DILU")])
+def test_march_f32(size, kind, precon):
     """The FP32 pass: a row is three products and three differences, and its
     error reaches the rows after it with the couplings of a diagonally
     dominant factor (a sum below one), so a few units of 2^-24 of the
     largest value, 64 allowed."""
-    c, rng, m, om = systems(size, "spd")
+    c, rng, m, om = systems(size, kind)
     r = rng.standard_normal(c.N)
-    w = m.precondition_f32("DIC", r).astype(np.float64)
-    ow = om.precondition("DIC", r.astype(np.float32).astype(np.float64))
+    w = m.precondition_f32(precon, r).astype(np.float64)
+    ow = om.precondition(precon, r.astype(np.float32).astype(np.float64))
     assert np.abs(w - ow).max() <= 64 * 2.0**-24 * np.abs(ow).max()
 
 
