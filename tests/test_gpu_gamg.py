@@ -557,24 +557,38 @@ def test_tile_dic_apply_variants(apply, shape, monkeypatch):
     assert np.abs(b - om.Amul(psi)).sum() / perf.normFactor < 1e-8
 
 
-@pytest.mark.parametrize("shape", [(16, 16, 16), (16, 17, 15), (32, 1, 3), (48, 40, 37),
-                                   (37, 40, 21), (144, 130, 113)])
+@pytest.mark.parametrize("shape", [(16, 16, 16), (16, 17, 15), (32, 2, 3), (16, 16, 2),
+                                   (48, 40, 37), (37, 40, 21), (144, 130, 113)])
 def test_tile_dic_in_registers(shape, monkeypatch):
-    """The symmetric tile-local DIC with the tile in registers: one tile, one
-    row or plane of a tile, partial tiles in every direction, and more tiles
-    than stay resident at once.  Its operations and their order are those of
-    the tile staged in LDS, so the results are the same bits."""
+    """The symmetric tile-local DIC with the tile in registers: one tile, few
+    rows or planes of a tile, partial tiles in every direction, and more
+    tiles than stay resident at once.  Its operations and their order are
+    those of the tile staged in LDS, so the results are the same bits.  In a
+    solve it also sums w.r and r: three iterations from either kernel differ
+    by the order of those FP64 sums, which can turn a rounding of the FP32
+    step lengths and with it of every vector (64 units of 2^-24 allowed); on
+    one tile there is one sum, in the same order."""
     nx, ny, nz = shape
     n, lower, upper = box(nx, ny, nz)
     rng = np.random.default_rng(29)
     diag, up = spd_coeffs(n, lower, upper, rng)
-    m = fh.lduMatrix(fh.lduAddressing(n, lower, upper), diag, up)
-    r = rng.standard_normal(n)
-    monkeypatch.setenv("FOAMHIP_TILE_APPLY", "lds")
-    w_lds = m.precondition_f32("tileDIC", r)
-    monkeypatch.setenv("FOAMHIP_TILE_APPLY", "regs")
-    w = m.precondition_f32("tileDIC", r)
-    assert np.array_equal(w, w_lds)
+    mesh = fh.lduAddressing(n, lower, upper)
+    assert mesh.info()["tiled"]
+    m = fh.lduMatrix(mesh, diag, up)
+    r, b = rng.standard_normal(n), rng.uniform(-1, 1, n)
+    ctl = {"solver": "PCG", "preconditioner": "DIC", "tolerance": 0, "relTol": 0, "maxIter": 3,
+           "precision": "mixed"}
+    w, x = {}, {}
+    for apply in ("lds", "regs"):
+        monkeypatch.setenv("FOAMHIP_TILE_APPLY", apply)
+        w[apply] = m.precondition_f32("tileDIC", r)
+        x[apply] = np.zeros(n)
+        perf = fh.solver_New("p", m, ctl).solve(x[apply], b)
+        assert perf.nIterations == 3 and perf.finalResidual < perf.initialResidual
+    assert np.array_equal(w["regs"], w["lds"])
+    if max(shape) <= 16:
+        assert np.array_equal(x["regs"], x["lds"])
+    assert np.abs(x["regs"] - x["lds"]).max() <= 64 * 2.0**-24 * np.abs(x["lds"]).max()
 
 
 AGG_CASES = [
