@@ -230,3 +230,71 @@ def test_h_device_matches_host(case):
         fh._check(fh.lib().fh_face_h_device(m.handle, nc, P(d_x), P(d_f)))
         np.testing.assert_array_equal(host(d_h), m.H(X).reshape(-1))
         np.testing.assert_array_equal(host(d_f), m.faceH(X).reshape(-1))
+
+
+def test_work_arrays_between_calls():
+    """H of one, nine, one and three components between assemblies, coefficient
+    updates and a larger number of components on the same matrix: the work
+    arrays they share give every call its own result."""
+    c = BoxCase(11, 7, 5)
+    rng = np.random.default_rng(61)
+    a = O.Addr(c.N, c.lower, c.upper)
+    mesh = fh.lduAddressing(c.N, c.lower, c.upper)
+    bnd = fh.Boundary(mesh, c.bFaceCells)
+    m = fh.lduMatrix(mesh)
+    d_ic = torch.empty(c.nB, dtype=torch.float64, device="cuda")
+    d_bc = torch.empty_like(d_ic)
+    for k, nc in enumerate((1, 9, 1, 3)):
+        phi, bPhi = c.fourier_flux(3 + k)
+        diag, upper, lower, _, _ = O.convection_diffusion(a, c, phi, bPhi, 0.1)
+        if k % 2 == 0:
+            ins = [dev(phi)] + [dev(c.magSf), dev(c.deltaCoeffs), dev(bPhi), dev(c.bMagSf),
+                                dev(c.bDeltaCoeffs), dev(c.bType, np.int32), dev(c.bValue)]
+            torch.cuda.synchronize()
+            fh._check(fh.lib().fh_assemble_convection_diffusion(
+                m.handle, bnd.handle, P(ins[0]), ctypes.c_double(0.1), *[P(t) for t in ins[1:]],
+                P(d_ic), P(d_bc), None, 0))
+        else:
+            m.set(diag, upper[:c.F], lower[:c.F])
+        X = rng.standard_normal((c.N, nc))
+        d_x, d_h = dev(X), torch.empty(c.N * nc, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        fh._check(fh.lib().fh_h_device(m.handle, nc, P(d_x), P(d_h)))
+        om = O.Matrix(a, diag, upper[:c.F], lower[:c.F])
+        ref = np.stack([om.H(X[:, q].copy()) for q in range(nc)], 1)
+        np.testing.assert_array_equal(host(d_h), ref.reshape(-1))
+        np.testing.assert_array_equal(m.coeffs()[0], diag)
+
+
+def test_gradients_from_two_threads():
+    """Gradients on one mesh from two threads, twenty each, share its face
+    work: each result is its own field's."""
+    import threading
+    c = BoxCase(31, 17, 13)
+    rng = np.random.default_rng(71)
+    a = O.Addr(c.N, c.lower, c.upper)
+    mesh = fh.lduAddressing(c.N, c.lower, c.upper)
+    bnd = fh.Boundary(mesh, c.bFaceCells)
+    geo = [dev(c.weights), dev(c.Sf), dev(c.V), dev(c.bSf), dev(c.bMagSf)]
+    bad = []
+
+    def run(seed):
+        r = np.random.default_rng(seed)
+        phi, bPhi, bSn = (r.standard_normal(k) for k in (c.N, c.nB, c.nB))
+        ref = O.grad_gauss_linear(a, phi, c.weights, c.Sf, c.V, c.bFaceCells, c.bSf, c.bMagSf,
+                                  bPhi, bSn)
+        ins = [dev(phi)] + geo + [dev(bPhi), dev(bSn)]
+        out = [torch.empty(3 * k, dtype=torch.float64, device="cuda") for k in (c.N, c.nB)]
+        torch.cuda.synchronize()
+        for _ in range(20):
+            st = fh.lib().fh_grad_gauss_linear(mesh.handle, bnd.handle, *[P(t) for t in ins],
+                                               *[P(t) for t in out])
+            if st or not all(np.array_equal(host(o), e) for o, e in zip(out, ref)):
+                bad.append((seed, st))
+
+    threads = [threading.Thread(target=run, args=(s,)) for s in (1, 2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
