@@ -1220,7 +1220,14 @@ __device__ __forceinline__ void vf_rows(const RowsView& R, const SweepData<T>& d
     {
         if (KIND == SWEEP_PRECOND_FWD) a = b*a;
 #pragma unroll
-        for (int m = 0; m < M; m++) val[m] = m < nDep ? b*val[m] : T(0);   // (b may be infinite)
+        for (int m = 0; m < M; m++) val[m] = b*val[m];
+        // (an infinite or NaN factor must not reach the slots past the row's)
+        if (__any(!(b - b == T(0))))
+        {
+#pragma unroll
+            for (int m = 0; m < M; m++)
+                if (m >= nDep) val[m] = T(0);
+        }
     }
     // ---- the wait ----
     auto late = [&] {
