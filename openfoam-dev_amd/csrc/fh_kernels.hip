@@ -744,8 +744,9 @@ void k_sweep_parts(RowsView R, SchedView S, SweepSync sync, SweepData<T> d,
     if (expired && st) st->scheduleError = 1;
 }
 
-// A row of the chunk sweep in two halves, for the Gauss-Seidel and the
-// DIC/DILU application kinds.  Before the chunk's wait: the row's shape and
+// A row of the chunk sweep that waits on chunk flags (k_sweep_chunks) in two
+// halves, for the Gauss-Seidel and the DIC/DILU application kinds (with
+// FOAMHIP_CHUNK_SYNC=flags; by default they poll values, further down).  Before the chunk's wait: the row's shape and
 // scalars (source and diagonal, or rD and x / the forward result), the
 // columns and coefficients of its first ROW_PREFETCH entries (32: with 16,
 // the coarse GAMG levels' longer rows loaded their last entries one by one
@@ -835,12 +836,6 @@ template<> struct SweepSentinel<float>
     __device__ static bool is(float v) { return __float_as_int(v) == bits; }
 };
 
-// A row's entries past the prefetched ones, [kLo, kHi), 16 at a time with
-// every load of a block in flight (columns and coefficients, then the
-// values): ascending for Gauss-Seidel and the forward pass, descending for
-// the backward pass.  Dependency values come from wDep (with VF: polled
-// until no longer the sentinel), the others from wIn.  acc -= c*w
-// (Gauss-Seidel) or acc -= rD*c*w.
 // where the values of the sweep are polled: the output in memory, or a copy
 // of the whole vector in LDS (one workgroup sweeps the mesh)
 template<class T>
@@ -872,6 +867,12 @@ struct VfLds
     }
 };
 
+// A row's entries past its registers, [kLo, kHi), 16 at a time with
+// every load of a block in flight (columns and coefficients, then the
+// values): ascending for Gauss-Seidel and the forward pass, descending for
+// the backward pass.  Dependency values come from wDep (with VF: polled
+// until no longer the sentinel), the others from wIn.  acc -= c*w
+// (Gauss-Seidel) or acc -= rD*c*w.
 template<class T, int KIND, bool BACKWARD, bool VF, class W>
 __device__ __forceinline__ T row_tail(const RowsView& R, const SweepData<T>& d, const T* wIn,
                                       const W& wDep, int32_t base, int32_t nLo, int32_t kLo,
@@ -1105,6 +1106,9 @@ void k_sweep_chunks(RowsView R, SweepData<T> d, ChunkView C, RowSync sync,
 // with an obstacle): 204 us forward, 217 backward, 0.95 us a level, which is
 // one hand-off through memory; with one lane polling the latest dependency
 // before the rows loaded theirs, and 32 slots for every row, 564 and 606.
+// (Not excluded as a part of it: the four slot widths are one kernel of 217
+// to 256 registers in FP64, with 106 to 250 scalar registers, mostly masks,
+// spilled into lanes of vector registers.)
 //
 // Polling every dependency multiplies the loads of a level by the rounds of
 // polling, which pays while they are few.  With 32 slots, or where the
@@ -1406,6 +1410,8 @@ void k_sweep_chunks_vf(RowsView R, SweepData<T> d, const T* wIn, T* wOut, ChunkV
 // wavefront, 0.33 us for DIC rows of one dependency, 0.6 for 8 to 15, 0.8
 // with a Gauss-Seidel row's other side (4, 8 and 12 wavefronts measured the
 // same until registers spilled; raised priority past the gate took 0.1 off).
+// (The four slot widths are one kernel here too, 122 to 188 registers in FP64
+// and 11 to 123 scalar registers spilled: 84 in the Gauss-Seidel forward one.)
 // Gauss-Seidel sweeps of the coarse levels of a 64 x 48 x 48 GAMG hierarchy
 // (us, before: one workgroup with a barrier per level, or through memory
 // from 16 rows a level on): 17756 rows in 315 levels 376 (489), 4431 in 197

@@ -1115,7 +1115,7 @@ __device__ __forceinline__ tl_f4 tl_h4(tl_u2 v)
 // What bounds it: a step is about 50 instructions of one wavefront per SIMD
 // (the registers allow no second one), and the code is about 42 KB, fetched
 // by every CU in every launch.  Measured at 256^3 (4096 tiles): 106 us, 2.8
-// TB/s of the 302 MB it has to move, against 146 us for the row walk and 167
+// TB/s of the 302 MB it has to move (307 counted), against 146 us for the row walk and 167
 // us for the staged tile (59 KB of LDS allow two tiles per CU, the registers
 // four); 32^3: 14 us against 18 staged.  Loading plane by plane (slots
 // turned by j + q, twice the selects) measured 133 us.

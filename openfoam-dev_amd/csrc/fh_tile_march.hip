@@ -9,8 +9,11 @@
 // coordinates), and each row keeps the reference face order (k, j, i), so
 // the results are bitwise those of the sequential loops.
 //
-// What bounds such a pass is the chain of dependent cells, not the traffic.
-// A workgroup therefore owns a pencil of 16 x 16 columns and marches along
+// What bounds such a pass is first the chain of dependent cells, then what a
+// compute unit can load: most of the chain is the lag between the starts of
+// the pencils, and where the packed coefficients come from HBM (they do in a
+// solve of a box beyond the last-level cache) a pass takes about a quarter
+// longer than launched back to back.  A workgroup therefore owns a pencil of 16 x 16 columns and marches along
 // k through the whole box without stopping: four wavefronts compute (16
 // columns along i by 4 along j each, lane (i, j) at plane k = step - i -
 // 2 j), so the chain has nz + 21 steps per wavefront and no tile to drain
@@ -39,13 +42,17 @@
 // Pencils are taken by ticket along their diagonals, so every pencil waited
 // on is already running; every wait is bounded.
 //
-// Measured on an MI355X against the 8 x 8 x 16 tiles of fh_tile_wave.hip
-// (us per pass, forward / backward with its sum):
-//                      FP64 here   tiles       FP32 here   tiles
-//     64^3             70 / 76     130 / 136   56 / 62     118 / 128
-//     128^3            152 / 163   288 / 302   121 / 131   286 / 307
-//     200 x 150 x 133  208 / 222   382 / 394   180 / 191   379 / 401
-//     256^3            493 / 520   641 / 652   342 / 375   604 / 640
+// Measured on an MI355X against the 8 x 8 x 16 tiles of fh_tile_wave.hip,
+// launched back to back, and in solves (kernel trace without the launches
+// past convergence; the 128^3 PBiCGStab's backward passes take no sum), us
+// per pass, forward / backward with its sum:
+//                      FP64 here   in a solve  tiles       FP32 here   tiles
+//     64^3             70 / 76     70 / 78     130 / 136   56 / 62     118 / 128
+//     128^3            152 / 163   193 / 188   288 / 302   121 / 131   286 / 307
+//     200 x 150 x 133  208 / 222   273 / 285   382 / 394   180 / 191   379 / 401
+//     256^3            493 / 520               641 / 652   342 / 375   604 / 640
+// (256^3: 978 and 956 MB of traffic counted, 804 and 938 read or written
+// once: the skew's padding and the halos.)
 // A Gauss-Seidel row also takes the values on its other side, which the
 // sweep does not change before the row is reached (forward: old ones) or at
 // all (backward: the forward pass's).  Forward their three products are
@@ -61,6 +68,8 @@
 //     256 x 256 x 16   393 / 657     611 / 1188
 //     200 x 150 x 133  565 / 878     1035 / 1955
 //     256^3            1390 / 2035   2435 / 4350
+// (in a solve of 150 x 100 x 60 cells the two kernels alone take 188 and 154
+// us, back to back 161 and 134).
 // A step takes 0.10 (FP32) to 0.16 us (FP64) in a pencil alone, where a
 // compute unit moves 60 to 80 GB/s; a pencil starts about 20 (i) or 47 (j)
 // steps and one hand-off through memory after the one before.
@@ -709,10 +718,10 @@ void k_sweep_march(MarchArgs<T> A, DevState* st, FusedFinalize F)
 // rD (forward) and the three coefficients times it; Gauss-Seidel: the
 // coefficients and the diagonal (rD); OLD: the coefficients times rD (psi)
 // at the neighbour on the other side.
-// A workgroup writes one value of 64 steps of one wavefront: it reads the planes these steps touch as rows of 16 cells and turns them
-// into steps in LDS.  (Read in step order every lane is in another plane:
-// with that the products of a 256^3 forward sweep took longer than the
-// sweep.)
+// A workgroup writes one value of 64 steps of one wavefront: it reads the
+// planes these steps touch as rows of 16 cells and turns them into steps in
+// LDS.  (Read in step order every lane is in another plane: with that the
+// products of a 256^3 forward sweep took longer than the sweep.)
 constexpr int MPS = 64;           // steps per workgroup
 template<class T, int MODE, bool OLD>
 __global__ __launch_bounds__(256)
