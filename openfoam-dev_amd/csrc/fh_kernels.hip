@@ -1225,8 +1225,12 @@ __device__ __forceinline__ void vf_rows(const RowsView& R, const SweepData<T>& d
         if (KIND == SWEEP_PRECOND_FWD) a = b*a;
 #pragma unroll
         for (int m = 0; m < M; m++) val[m] = b*val[m];
-        // (an infinite or NaN factor must not reach the slots past the row's)
-        if (__any(!(b - b == T(0))))
+        // (An infinite or NaN factor must not reach the slots past the row's.
+        // Said to be unlikely in FP32 alone: a DIC pass of the box above takes
+        // 202 / 226 us with that and 207 / 232 without, in FP64 212 / 237 and
+        // 213 / 231, by the compiler's order of what surrounds it.)
+        const bool inf = __any(!(b - b == T(0))) != 0;
+        if (sizeof(T) == 4 ? __builtin_expect(inf, 0) != 0 : inf)
         {
 #pragma unroll
             for (int m = 0; m < M; m++)
